@@ -28,24 +28,15 @@ static void rk_coeffs(int nrk, int irk, double& c1, double& c2) {
 // ---------------------------------------------------------------------------
 // kernel dispatch
 // ---------------------------------------------------------------------------
-// flux launch of one sweep with the grid's tile shape; the tiled variants
-// are instantiated for the WENO5 and PPM4 reconstructions
+// cells along x of a block of the y and z sweeps, for the tile rows 1, 2, 4
+// of echo_set_tile
+static int flux_tx(int ty) { return ty == 1 ? 16 : ty == 2 ? 32 : 8; }
+
+// flux launch of one sweep with the grid's tile shape
 template <int DIR, int REC, int SYS, bool ZZ>
 static void launch_flux_rec(echo_grid* g, double* partial) {
-  dim3 grid(g->nb[DIR - 1]), block(FLUX_BLOCK);
-  double* F = g->F[DIR - 1];
-  double* L = g->L[DIR - 1];
-  if constexpr (DIR > 1 && (REC == REC_WENO5 || REC == REC_PPM4)) {
-    if (g->tile[DIR - 1] == 2) {
-      k_flux<DIR, REC, SYS, ZZ, 2><<<grid, block, 0, g->stream>>>(g->ga, g->V, F, L, partial);
-      return;
-    }
-    if (g->tile[DIR - 1] == 4) {
-      k_flux<DIR, REC, SYS, ZZ, 4><<<grid, block, 0, g->stream>>>(g->ga, g->V, F, L, partial);
-      return;
-    }
-  }
-  k_flux<DIR, REC, SYS, ZZ, 1><<<grid, block, 0, g->stream>>>(g->ga, g->V, F, L, partial);
+  k_flux<DIR, REC, SYS, ZZ><<<g->nb[DIR - 1], FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, g->F[DIR - 1], g->L[DIR - 1],
+                                                                          partial, flux_tx(g->tile[DIR - 1]));
 }
 
 template <int DIR, int SYS, bool ZZ>
@@ -63,8 +54,10 @@ static void launch_flux_dir(echo_grid* g, double* partial) {
 
 // launch blocks of a sweep for tile shape ty (padded for xcd_block)
 static unsigned flux_blocks(const echo_config& c, int d, int ty) {
-  long long t = d == 0 ? flux_tiles<1>(c.nx, c.ny, c.nz, 1)
-              : d == 1 ? flux_tiles<2>(c.nx, c.ny, c.nz, ty) : flux_tiles<3>(c.nx, c.ny, c.nz, ty);
+  const int tx = flux_tx(ty);
+  long long t = d == 0 ? flux_tiles<1>(c.nx, c.ny, c.nz, tx, c.boundary_cond)
+              : d == 1 ? flux_tiles<2>(c.nx, c.ny, c.nz, tx, c.boundary_cond)
+                       : flux_tiles<3>(c.nx, c.ny, c.nz, tx, c.boundary_cond);
   return (unsigned)((t + NXCD - 1) / NXCD * NXCD);
 }
 

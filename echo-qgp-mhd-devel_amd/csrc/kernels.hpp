@@ -95,10 +95,10 @@ struct ImexView {
   int phase;              // 0: not inside an implicit stage
 };
 
-// 128 threads (two waves) per flux block: with 24 KB of LDS per block, six
-// blocks share a CU at three waves per SIMD, and the smaller blocks even out
-// the tail of a sweep (about 1% faster sweeps than 256)
-constexpr int FLUX_BLOCK = 128;
+// 256 threads (four waves) per flux block: 16 x 16 cells of a y or z sweep
+// own 15 rows of interfaces, one row of cells in sixteen is reconstructed by
+// two tiles
+constexpr int FLUX_BLOCK = 256;
 constexpr int UPDATE_BLOCK = 256;
 constexpr int FIX_BLOCK = 256;
 constexpr int NXCD = 8;   // MI355X: 8 XCDs, each with its own L2
@@ -158,142 +158,277 @@ __device__ __forceinline__ int bc_map(int c0, int m, int bc) {
 }
 
 // ---------------------------------------------------------------------------
-// k_flux: one thread per interface normal to DIR.  Reconstructs the nv
-// primitives (WENO5/PPM4/TVD2/...) from the six cells around the interface,
-// applies the reference's repair of unphysical states (evolve.f90:334-369),
-// evaluates the HLL flux (work.f90:195-229 with system_flux of
-// system.f90:1316-1583) and writes it, plus a per-block max of the fast
-// speeds for the CFL condition (evolve.f90:723-764).
+// k_flux: HLL fluxes on the interfaces normal to DIR.  One thread per cell of
+// a tile: it reconstructs the nv primitives of its cell at both of the cell's
+// faces (WENO5/PPM4/TVD2/...; from the five cells around it), hands the lower
+// one to the thread of the cell below through LDS, and then owns the cell's
+// upper interface: the reference's repair of unphysical states
+// (evolve.f90:334-369), the HLL flux (work.f90:195-229 with system_flux of
+// system.f90:1316-1583), and a per-block max of the fast speeds for the CFL
+// condition (evolve.f90:723-764).
+//
+// What bounds it: FP64 VALU issue (some 4 cycles per wave instruction, with
+// two or three waves per SIMD).  Reconstructing by cell instead of by
+// interface shares the smoothness indicators between a cell's two faces and
+// loads five cells per variable instead of six; the price is one row of
+// cells per tile whose upper face the next tile owns.
 // ---------------------------------------------------------------------------
 //
-// Tile shape (TY): with TY = 1 a block takes FLUX_BLOCK consecutive faces in
-// the face order (x fastest).  For the y and z sweeps TY > 1 makes the block
-// a tile of FLUX_BLOCK/TY faces along x by TY faces along the sweep, so the
-// six-cell stencils of the block's faces overlap in TY + 5 cell rows instead
-// of 6 * TY; the autotuner picks TY per sweep and grid.
+// Tiles.  x sweep: the cells -1 .. nx of every row (the ghost cells included)
+// lie in one sequence of slots, a block takes FLUX_BLOCK slots and the
+// FLUX_BLOCK - 1 interfaces between them (interfaces across the end of a row
+// do not exist).  y and z sweeps: a block is TX cells along x by FLUX_BLOCK/TX
+// cells along the sweep, and owns one interface row less than cell rows.
+// `tx` is the TX of the launch (a power of two): fewer columns mean more rows
+// and so a smaller share of cells that two tiles reconstruct, and shorter
+// pieces of a cache line per row.
+constexpr int FLUX_TX_MAX = 32;
+constexpr int FLUX_STAGE = FLUX_BLOCK + 4 * FLUX_TX_MAX;   // staged cells of a tile
+// ghost cells per end of a row in the slots of an x sweep: outflow needs the
+// one whose interface states enter a flux (the stencil's other cells outside
+// are copies of the row's end), periodic rows need three
+__host__ __device__ __forceinline__ int flux_ghosts(int bc) { return bc == 0 ? 3 : 1; }
+
 template <int DIR>
-__host__ __device__ __forceinline__ long long flux_tiles(int nx, int ny, int nz, int ty) {
-  const long long nf = DIR == 1 ? (long long)(nx + 1) * ny * nz
-                     : (DIR == 2 ? (long long)nx * (ny + 1) * nz : (long long)nx * ny * (nz + 1));
-  if (ty == 1 || DIR == 1) return (nf + FLUX_BLOCK - 1) / FLUX_BLOCK;
-  const int tx = FLUX_BLOCK / ty;
+__host__ __device__ __forceinline__ long long flux_tiles(int nx, int ny, int nz, int tx, int bc) {
+  if (DIR == 1)
+    return ((long long)(nx + 2 * flux_ghosts(bc)) * ny * nz - 1 + FLUX_BLOCK - 2) / (FLUX_BLOCK - 1);
+  const int rows = FLUX_BLOCK / tx - 1;
   const long long ntx = (nx + tx - 1) / tx;
-  const long long nti = ((DIR == 2 ? ny : nz) + 1 + ty - 1) / ty;
+  const long long nti = ((DIR == 2 ? ny : nz) + 1 + rows - 1) / rows;
   return ntx * nti * (DIR == 2 ? nz : ny);
 }
 
-// Launch bounds (FLUX_BLOCK, 3): at most 168 VGPRs, so three waves share
-// each SIMD.  Unbounded, the viscous WENO5 kernel takes 320 VGPRs (one wave
-// per SIMD) and its FP64 chains and stencil loads stall with nothing to
-// switch to.  The reconstructed states are what does not fit: 2 x NV doubles
-// per lane beside the stencils in flight and the side states.  They wait in
-// LDS instead, sw[2][NV][FLUX_BLOCK] (24 KB per block for NV = 12: 144 KB
-// for the six blocks of a CU at three waves per SIMD).  In viscous runs the pi^{mu nu} components go there as
-// soon as they are reconstructed; rho, v and p stay in registers for the
-// repair.  Each lane touches only its own column of sw, so no barrier is
-// needed.  Every variant then fits without scratch spills; before this, the
-// viscous WENO5 kernel spilled ~48 VGPRs per lane to scratch, which lives in
-// HBM (about 1.7 GB of extra traffic per sweep on 192 x 192 x 128).  The
-// viscous resistive system (NV = 19, 39 KB of LDS per block) fits four
-// blocks per CU, two waves per SIMD, and is bounded for that.
+// components staged at a time
+template <int SYS>
+constexpr int flux_group() {
+  return SysT<SYS>::NV == 5 || SYS == SYS_MHDGLM ? 5 : 4;
+}
+
+// Launch bounds: three waves per SIMD (at most 168 VGPRs); 49 KB of LDS per
+// block for NV = 12 (three blocks per CU).  The viscous resistive system
+// (NV = 19, 64 KB per block) fits two blocks per CU, two waves per SIMD, and
+// is bounded for that.
 template <int SYS>
 constexpr int flux_waves() { return SysT<SYS>::NV > 12 ? 2 : 3; }
 
-template <int DIR, int REC, int SYS, bool ZZ, int TY = 1>
+// barrier of the block that orders its LDS accesses only: loads from memory
+// stay in flight across it
+__device__ __forceinline__ void block_sync_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int DIR, int REC, int SYS, bool ZZ>
 __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs a, const double* __restrict__ V,
                                                      double* __restrict__ F, double* __restrict__ L,
-                                                     double* __restrict__ partial) {
+                                                     double* __restrict__ partial, int tx) {
   constexpr bool VISC = SysT<SYS>::VISC;
   constexpr int NV = SysT<SYS>::NV;
-  static_assert(TY == 1 || DIR != 1, "x sweeps use TY = 1");
   if (a.S->temp_check) return;   // the run has stopped (check_temp)
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const int m = DIR == 1 ? nx : (DIR == 2 ? ny : nz);
-  const long long nf = DIR == 1 ? (long long)(nx + 1) * ny * nz
-                     : (DIR == 2 ? (long long)nx * (ny + 1) * nz : (long long)nx * ny * (nz + 1));
-  const long long tile = xcd_block(blockIdx.x, gridDim.x);
-  long long f;
-  bool inside;
-  if constexpr (TY == 1) {
-    f = tile * FLUX_BLOCK + threadIdx.x;
-    inside = f < nf;
+  const unsigned t = threadIdx.x;
+  const unsigned tile = (unsigned)xcd_block(blockIdx.x, gridDim.x);
+  // the thread's cell: index ci along the sweep (-1 .. m), and whether it owns
+  // its upper interface, number ci + 1 of the line, f in the face array.
+  // Threads without a cell work on values of other cells up to the exchange.
+  int ci;
+  unsigned f;
+  long long base = 0, stride = 0;
+  bool owns;
+  unsigned w = 0, row0 = 0, q0 = 0, lg = 0;
+  int cfirst = 0;
+  const unsigned up = DIR == 1 ? 1u : (unsigned)tx;   // thread of the cell above
+  const int gh = flux_ghosts(a.bc);
+  if constexpr (DIR == 1) {
+    const unsigned rows = (unsigned)ny * (unsigned)nz;
+    w = (unsigned)(nx + 2 * gh);
+    const unsigned s0 = tile * (FLUX_BLOCK - 1u);
+    row0 = s0 / w;
+    q0 = s0 - row0 * w;
+    const unsigned q = q0 + t, dr = q / w, row = row0 + dr;
+    ci = (int)(q - dr * w) - gh;
+    owns = row < rows && ci >= -1 && ci < nx && t < FLUX_BLOCK - 1u;
+    f = (unsigned)(ci + 1) + ((unsigned)nx + 1u) * row;
   } else {
-    constexpr int TX = FLUX_BLOCK / TY;
-    const long long ntx = (nx + TX - 1) / TX;
-    const long long nti = (m + 1 + TY - 1) / TY;
-    const long long r = tile / ntx;
-    const int x = (int)(tile % ntx) * TX + (int)threadIdx.x % TX;
-    const int i = (int)(r % nti) * TY + (int)threadIdx.x / TX;
-    const long long rest = r / nti;   // z (y sweep) or y (z sweep)
-    inside = x < nx && i <= m && rest < (DIR == 2 ? nz : ny);
-    f = DIR == 2 ? x + (long long)nx * (i + (long long)(ny + 1) * rest)
-                 : x + (long long)nx * (rest + (long long)ny * i);
+    const unsigned TX = (unsigned)tx, TY = FLUX_BLOCK / TX;
+    const unsigned ntx = ((unsigned)nx + TX - 1u) / TX, nti = ((unsigned)m + TY - 1u) / (TY - 1u);
+    const unsigned r = tile / ntx, rest = r / nti;   // rest: z (y sweep) or y (z sweep)
+    const unsigned x0 = (tile - r * ntx) * TX + (t & (TX - 1u));
+    lg = 31 - __clz((int)TX);
+    const unsigned ty = t >> lg;
+    cfirst = (int)((r - rest * nti) * (TY - 1u)) - 1;
+    const int c = cfirst + (int)ty;
+    const unsigned other = (unsigned)(DIR == 2 ? nz : ny);
+    owns = x0 < (unsigned)nx && c < m && ty < TY - 1u && rest < other;
+    const unsigned x = x0 < (unsigned)nx ? x0 : (unsigned)nx - 1u, o = rest < other ? rest : other - 1u;
+    ci = c;
+    f = DIR == 2 ? x + (unsigned)nx * ((unsigned)(ci + 1) + ((unsigned)ny + 1u) * o)
+                 : x + (unsigned)nx * (o + (unsigned)ny * (unsigned)(ci + 1));
+    base = DIR == 2 ? (long long)o * ny * nx + x : (long long)o * nx + x;
+    stride = DIR == 2 ? nx : (long long)nx * ny;
   }
-  double amax = 0.;
-  if (inside) {
-    int x, y, z, i;
-    long long base, stride;
-    if constexpr (DIR == 1) {
-      i = (int)(f % (nx + 1)); long long r = f / (nx + 1); y = (int)(r % ny); z = (int)(r / ny);
-      base = ((long long)z * ny + y) * nx; stride = 1;
-    } else if constexpr (DIR == 2) {
-      x = (int)(f % nx); long long r = f / nx; i = (int)(r % (ny + 1)); z = (int)(r / (ny + 1));
-      base = (long long)z * ny * nx + x; stride = nx;
+  const unsigned nf = DIR == 1 ? ((unsigned)nx + 1u) * ny * nz
+                    : (DIR == 2 ? (unsigned)nx * ((unsigned)ny + 1u) * nz : (unsigned)nx * ny * ((unsigned)nz + 1u));
+  const DevScalars* S = a.S;
+  const Metric M = make_metric(a.coordinates, S->t);
+  // Staging.  The tile's cells with two more at either end of the sweep pass
+  // through LDS, GS components at a time (st, two buffers): every value is
+  // loaded from memory once per tile, the loads of the next group are in
+  // flight while this one is reconstructed, and the five cells of a thread's
+  // stencil are LDS reads.  sw: the lower states.  Thread t reads the lower
+  // states of thread t + up, and only it does, so after the last barrier it
+  // may also write there.
+  // In viscous runs the first four items are the Lorentz velocity (gamma,
+  // gamma v^i), reconstructed for deriv (evolve.f90:324-331, 371-374); it is
+  // formed once per staged cell.
+  constexpr int NU = VISC ? 4 : 0, NI = NV + NU;
+  constexpr int GS = flux_group<SYS>(), NG = (NI + GS - 1) / GS, NBUF = NG > 1 ? 2 : 1;
+  static_assert(!VISC || (GS == 4 && NG >= 4), "the Lorentz velocity's lower states wait in the last group's slots");
+  __shared__ double sw[NV][FLUX_BLOCK];
+  __shared__ double st[NBUF][GS][FLUX_STAGE];
+  const unsigned tr = t + up < FLUX_BLOCK ? t + up : t;
+  // staged positions: p = t and, for the first 4 * up threads, p = FLUX_BLOCK + t
+  const bool second = t < 4u * up;
+  long long offA, offB;
+  unsigned ps[5];   // positions of the stencil cells ci-2 .. ci+2
+  if constexpr (DIR == 1) {
+    const unsigned rows = (unsigned)ny * (unsigned)nz;
+    auto cell = [&](unsigned p) {   // slot s0 + p - 2
+      const unsigned q = q0 + p < 2u ? 0u : q0 + p - 2u;
+      const unsigned dr = q / w;
+      const unsigned r = row0 + dr < rows ? row0 + dr : rows - 1u;
+      return (long long)r * nx + bc_map((int)(q - dr * w) - gh, m, a.bc);
+    };
+    offA = cell(t);
+    offB = second ? cell(FLUX_BLOCK + t) : offA;
+    // outflow: stencil cells outside the row are its first or last cell
+    const int lo = a.bc == 0 ? -3 : 0, hi = a.bc == 0 ? nx + 2 : nx - 1;
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+      int c = ci - 2 + j;
+      c = c < lo ? lo : (c > hi ? hi : c);
+      ps[j] = (unsigned)((int)t + 2 + c - ci);
+    }
+  } else {
+    auto cell = [&](unsigned p) {
+      const int c = cfirst - 2 + (int)(p >> lg);
+      return base + stride * bc_map(c < m + 2 ? c : m + 2, m, a.bc);
+    };
+    offA = cell(t);
+    offB = cell(second ? FLUX_BLOCK + t : t);
+#pragma unroll
+    for (int j = 0; j < 5; j++) ps[j] = t + j * up;
+  }
+  double ra[GS], rb[GS] = {}, va[3], vb[3] = {};
+  auto load = [&](int g) {
+    // ties the loads of a group to this point of the program: the compiler
+    // would issue those of all groups at once and spill them
+    asm volatile("" : "+v"(offA), "+v"(offB));
+    if (VISC && g == 0) {
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const double* Vk = V + (long long)(KVX + k) * a.N;
+        va[k] = Vk[offA];
+      }
+      if (second) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) vb[k] = V[(long long)(KVX + k) * a.N + offB];
+      }
+      return;
+    }
+#pragma unroll
+    for (int q = 0; q < GS; q++) {
+      const int k = g * GS + q - NU;
+      if (k >= NV) break;
+      ra[q] = VISC && k >= KVX && k <= KVZ ? va[k - KVX] : V[(long long)k * a.N + offA];
+    }
+    if (second) {
+#pragma unroll
+      for (int q = 0; q < GS; q++) {
+        const int k = g * GS + q - NU;
+        if (k >= NV) break;
+        rb[q] = VISC && k >= KVX && k <= KVZ ? vb[k - KVX] : V[(long long)k * a.N + offB];
+      }
+    }
+  };
+  // c0: the cell left of the interface, used by the repair (KVX..KPR)
+  double wl[NV], wu[4], c0[5];
+  double dEface = 0.;   // resistive: E^d(right cell) - E^d(left cell), for div E
+  load(0);
+#pragma unroll
+  for (int g = 0; g < NG; g++) {
+    if (VISC && g == 0) {
+      auto lorentz = [&](const double* v, unsigned p) {
+        const double gl = rsqrt_nr(1. - v[0] * v[0] - v[1] * v[1] - M.g3 * (v[2] * v[2]));
+        st[0][0][p] = gl;
+        st[0][1][p] = gl * v[0];
+        st[0][2][p] = gl * v[1];
+        st[0][3][p] = gl * v[2];
+      };
+      lorentz(va, t);
+      if (second) lorentz(vb, FLUX_BLOCK + t);
     } else {
-      x = (int)(f % nx); long long r = f / nx; y = (int)(r % ny); i = (int)(r / ny);
-      base = (long long)y * nx + x; stride = (long long)nx * ny;
-    }
-    (void)x; (void)y; (void)z;
-    // interface i lies between cells i-1 and i (0-based); stencil cells i-3 .. i+2
-    long long off[6];
 #pragma unroll
-    for (int j = 0; j < 6; j++) off[j] = base + stride * bc_map(i - 3 + j, m, a.bc);
-
-    const DevScalars* S = a.S;
-    const Metric M = make_metric(a.coordinates, S->t);
-    if constexpr (VISC) {
-      // Lorentz-velocity reconstruction feeding deriv, evolve.f90:324-331,
-      // 371-374; done first so that its 42 temporaries are dead before the
-      // nv reconstructions below
-      double wd[4][6];
-#pragma unroll
-      for (int j = 0; j < 6; j++) {
-        const double vx = V[(long long)KVX * a.N + off[j]];
-        const double vy = V[(long long)KVY * a.N + off[j]];
-        const double vz = V[(long long)KVZ * a.N + off[j]];
-        const double gl = rsqrt_nr(1. - vx * vx - vy * vy - M.g3 * (vz * vz));
-        wd[0][j] = gl; wd[1][j] = gl * vx; wd[2][j] = gl * vy; wd[3][j] = gl * vz;
+      for (int q = 0; q < GS; q++) {
+        if (g * GS + q >= NI) break;
+        st[g % NBUF][q][t] = ra[q];
       }
-      const long long nfl = nf;
+      if (second) {
 #pragma unroll
-      for (int q = 0; q < 4; q++) {
-        double l, r;
-        rec_face<REC>(wd[q], l, r);
-        // outputs are streamed: non-temporal stores keep them from
-        // evicting the stencil rows that neighbouring blocks still read
-        __builtin_nontemporal_store(l + r, &L[q * nfl + f]);
+        for (int q = 0; q < GS; q++) {
+          if (g * GS + q >= NI) break;
+          st[g % NBUF][q][FLUX_BLOCK + t] = rb[q];
+        }
       }
     }
-    // c0: the cell left of the interface, used by the repair (KVX..KPR).
-    // Components k >= KREG of wl, wr go straight to sw.
-    __shared__ double sw[2][NV][FLUX_BLOCK];
-    constexpr int KREG = VISC ? KPR + 1 : NV;
-    double wl[NV], wr[NV], c0[5];
-    double dEface = 0.;   // resistive: E^d(right cell) - E^d(left cell), for div E
+    if (g + 1 < NG) load(g + 1);
+    block_sync_lds();
+    if (VISC && g == 1) {
+      if (owns) {
 #pragma unroll
-    for (int k = 0; k < NV; k++) {
-      double s[6];
-      const double* Vk = V + (long long)k * a.N;
+        for (int q = 0; q < 4; q++)
+          // outputs are streamed: non-temporal stores keep them from
+          // evicting the rows that neighbouring blocks still read
+          __builtin_nontemporal_store(wu[q] + sw[NV - 4 + q][tr], &L[(long long)q * nf + f]);
+      }
+    }
 #pragma unroll
-      for (int j = 0; j < 6; j++) s[j] = Vk[off[j]];
-      double l, r;
-      rec_face<REC>(s, l, r);
-      if (k < KREG) { wl[k] = l; wr[k] = r; } else { sw[0][k][threadIdx.x] = l; sw[1][k][threadIdx.x] = r; }
+    for (int q = 0; q < GS; q++) {
+      const int it = g * GS + q, k = it - NU;
+      if (it >= NI) break;
+      double s[5], h, l;
+#pragma unroll
+      for (int j = 0; j < 5; j++) s[j] = st[g % NBUF][q][ps[j]];
+      rec_cell<REC>(s, h, l);
+      // h is used below only by the threads that own an interface: without
+      // this the compiler moves its arithmetic there and keeps the inputs
+      asm volatile("" : "+v"(h));
+      if (k < 0) {
+        wu[it] = h;
+        sw[NV - 4 + it][t] = l;   // rewritten two barriers after it was read
+        continue;
+      }
+      wl[k] = h;
+      sw[k][t] = l;
       if (k <= KPR) c0[k] = s[2];
       if constexpr (SysT<SYS>::RES) {
         if (k == SysT<SYS>::KE + DIR - 1) dEface = s[3] - s[2];
       }
     }
+  }
+  block_sync_lds();
+  // the left states of the first NPK components wait in the staging buffers
+  constexpr int NPK = NV < NBUF * GS * FLUX_STAGE / FLUX_BLOCK ? NV : NBUF * GS * FLUX_STAGE / FLUX_BLOCK;
+  static_assert(NPK > KPR, "the fluid's left states are parked");
+  double* pk = &st[0][0][0] + t;
+  double amax = 0.;
+  if (owns) {
+    double wr[5];
+#pragma unroll
+    for (int k = 0; k < 5; k++) wr[k] = sw[k][tr];
     // repair of reconstructed states with the cell left of the interface
     // (evolve.f90:334-369; the reference uses w0(ix) for both sides)
     {
@@ -323,48 +458,33 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
     if constexpr (SysT<SYS>::GLM) {
       // work_glm{x,y,z}, work.f90:67-139: Dedner interface values of psi and
       // the normal B.  The reference sets wr(psi) = wl(psi) before taking
-      // their difference, so the B update reduces to the average.  In the
-      // viscous resistive system these components wait in LDS.
+      // their difference, so the B update reduces to the average.
       constexpr int KB = SysT<SYS>::KB + DIR - 1, KG = SysT<SYS>::KG;
       const double ch = S->glm_ch;
-      double gl, gr, bl, br;
-      if constexpr (KG < KREG) { gl = wl[KG]; gr = wr[KG]; bl = wl[KB]; br = wr[KB]; }
-      else {
-        gl = sw[0][KG][threadIdx.x]; gr = sw[1][KG][threadIdx.x];
-        bl = sw[0][KB][threadIdx.x]; br = sw[1][KB][threadIdx.x];
-      }
-      gl = 0.5 * (gl + gr) - (br - bl) * ch / 2;
-      gr = gl;
-      bl = 0.5 * (bl + br) - (gr - gl) / (2 * ch);
-      br = bl;
-      if constexpr (KG < KREG) { wl[KG] = gl; wr[KG] = gr; wl[KB] = bl; wr[KB] = br; }
-      else {
-        sw[0][KG][threadIdx.x] = gl; sw[1][KG][threadIdx.x] = gr;
-        sw[0][KB][threadIdx.x] = bl; sw[1][KB][threadIdx.x] = br;
-      }
+      const double gl = wl[KG], gr = sw[KG][tr], bl = wl[KB], br = sw[KB][tr];
+      const double g = 0.5 * (gl + gr) - (br - bl) * ch / 2, bm = 0.5 * (bl + br);
+      wl[KG] = g; sw[KG][tr] = g;
+      wl[KB] = bm; sw[KB][tr] = bm;
     }
-    // Park wr in LDS while the left side state is formed, then wl while the
-    // right one is.  side_state completes the pi^{tau mu} components of its
-    // input (derived_pi), so each side is stored after its own side_state.
-    // The empty asm statements with a memory clobber keep the compiler from
-    // forwarding the stored values in registers across the side-state
-    // computations, which is what would spill.
+    // The right states wait in LDS while the left side state is formed, the
+    // left ones while the right one is.  side_state completes the pi^{tau mu}
+    // components of its input (derived_pi), so each side is stored after its
+    // own side_state.  The empty asm statements with a memory clobber keep the
+    // compiler from forwarding the stored values in registers across the
+    // side-state computations, which is what would spill.
 #pragma unroll
-    for (int k = 0; k < KREG; k++) sw[1][k][threadIdx.x] = wr[k];
-#pragma unroll
-    for (int k = KREG; k < NV; k++) wl[k] = sw[0][k][threadIdx.x];
+    for (int k = KVX; k <= KPR; k++) sw[k][tr] = wr[k];
     SideState sl, sr;
     int e = side_state<DIR, SYS, ZZ>(a.eos, M, wl, sl);
 #pragma unroll
-    for (int k = 0; k < NV; k++) sw[0][k][threadIdx.x] = wl[k];
+    for (int k = 0; k < NPK; k++) pk[k * FLUX_BLOCK] = wl[k];
     asm volatile("" ::: "memory");
     {
       double wv[NV];
 #pragma unroll
-      for (int k = 0; k < NV; k++) wv[k] = sw[1][k][threadIdx.x];
+      for (int k = 0; k < NV; k++) wv[k] = sw[k][tr];
       if (e == 0) e = side_state<DIR, SYS, ZZ>(a.eos, M, wv, sr);
-#pragma unroll
-      for (int k = 0; k < NV; k++) sw[1][k][threadIdx.x] = wv[k];
+      if constexpr (VISC && ZZ) sw[KPIZZ][tr] = wv[KPIZZ];
     }
     asm volatile("" ::: "memory");
     if (e != 0) {
@@ -392,15 +512,15 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
       for (int k = 0; k < NV; k++) {
         double ql[NV], qr[NV];
 #pragma unroll
-        for (int j = 0; j < NV; j++) { ql[j] = sw[0][j][threadIdx.x]; qr[j] = sw[1][j][threadIdx.x]; }
-        double ulk = u_comp<SYS>(k, M, sl, ql) * M.gp;
-        double urk = u_comp<SYS>(k, M, sr, qr) * M.gp;
-        double flk = f_comp<DIR, SYS>(k, M, sl, ql) * M.gp;
-        double frk = f_comp<DIR, SYS>(k, M, sr, qr) * M.gp;
+        for (int j = 0; j < NV; j++) { ql[j] = j < NPK ? pk[j * FLUX_BLOCK] : wl[j]; qr[j] = sw[j][tr]; }
+        double ulk = u_comp<SYS>(k, M, sl, ql);
+        double urk = u_comp<SYS>(k, M, sr, qr);
+        double flk = f_comp<DIR, SYS>(k, M, sl, ql);
+        double frk = f_comp<DIR, SYS>(k, M, sr, qr);
         double fk;
         if (SysT<SYS>::RES && k >= SysT<SYS>::KB) fk = 0.5 * (flk + frk - clight * (urk - ulk));
         else fk = a1 * (ap * flk + am * frk - ap * am * (urk - ulk));
-        __builtin_nontemporal_store(fk, &F[(long long)k * nf + f]);
+        __builtin_nontemporal_store(fk * M.gp, &F[(long long)k * nf + f]);
       }
       if constexpr (SysT<SYS>::RES) __builtin_nontemporal_store(dEface, &F[(long long)NV * nf + f]);
     }
@@ -409,9 +529,9 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
   __shared__ double red[FLUX_BLOCK / 64];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) amax = dmax(amax, __shfl_xor(amax, o, 64));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+  if ((t & 63) == 0) red[t >> 6] = amax;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     double r = red[0];
 #pragma unroll
     for (int w = 1; w < FLUX_BLOCK / 64; w++) r = dmax(r, red[w]);

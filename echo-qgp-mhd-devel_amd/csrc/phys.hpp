@@ -61,14 +61,15 @@ struct Eos {
 
 struct Metric {
   double g1, g2, g3, gp, gm, g0, t;
+  double ig3;   // 1 / g3: the flux path multiplies by it (a division is ten instructions per lane)
 };
 
 __host__ __device__ __forceinline__ Metric make_metric(int coordinates, double t) {
   // system_metric_minkowski / _bjorken, system.f90:132-160
   Metric m;
   m.g1 = 1.; m.g2 = 1.; m.g0 = -1.; m.t = t;
-  if (coordinates == BJORKEN) { m.g3 = t * t; m.gp = t; m.gm = 1. / t; }
-  else { m.g3 = 1.; m.gp = 1.; m.gm = 1.; }
+  if (coordinates == BJORKEN) { m.g3 = t * t; m.gp = t; m.gm = 1. / t; m.ig3 = 1. / m.g3; }
+  else { m.g3 = 1.; m.gp = 1.; m.gm = 1.; m.ig3 = 1.; }
   return m;
 }
 
@@ -240,33 +241,31 @@ __host__ __device__ __forceinline__ int get_derived_data(const Eos& E, double rh
   return 0;
 }
 
-// 1/x for finite x > 0 in the normal range: the hardware reciprocal and two
-// Newton-Raphson steps, within about an ulp of the correctly rounded value,
-// in five instructions instead of the ten of the IEEE division sequence.
+// 1/x for finite x > 0 in the normal range: the hardware reciprocal (relative
+// error e below 2^-22) and one cubic step r (1 + e + e^2), whose error e^3 is
+// below the rounding, in four instructions instead of the ten of the IEEE
+// division sequence.
 __device__ __forceinline__ double rcp_nr(double x) {
-  double r = __builtin_amdgcn_rcp(x);
-  double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
 // 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
-// hardware reciprocal square root and two Newton-Raphson steps, within about
-// an ulp of 1/sqrt(x); x = 0 gives +inf as the IEEE form does.
+// hardware reciprocal square root and one cubic step r (1 + e/2 + 3 e^2/8),
+// e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
 __device__ __forceinline__ double rsqrt_nr(double x) {
-  double r = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  double e = __builtin_fma(-h * r, r, 0.5);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-h * r, r, 0.5);
-  r = __builtin_fma(r, e, r);
-  return x == 0.0 ? __builtin_inf() : r;
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * r), r, 1.0);
+  const double y = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
+  return x == 0.0 ? __builtin_inf() : y;
 }
 
 // ---------------------------------------------------------------------------
-// Reconstruction (holib.f90).  f[0..5] = cells i-2 .. i+3 around the
-// interface i+1/2; returns the left (gl) and right (gr) states there.
+// Reconstruction (holib.f90), by cell: f[0..4] = cells c-2 .. c+2; hi is the
+// state at the cell's upper face (the left state of interface c+1/2), lo the
+// one at its lower face (the right state of interface c-1/2).  A scheme's two
+// sides of an interface mirror each other, so lo is hi of the mirrored cells.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double sgn1(double d) { return copysign(1.0, d); }
 
@@ -310,28 +309,34 @@ __device__ __forceinline__ double mp5(double f, double f1, double f2, double f3,
   return r;
 }
 
-// One WENO5 side (holib.f90:206-217).  The reference's weights
-// alpha_k = d_k / (beta_k/12 + eps)^2, normalised by their sum, are
-// evaluated as  w_k = d_k * prod_{j != k} Q_j  with Q_j = (beta_j + 12 eps)^2:
-// the same ratios (the factor 144 cancels), with one reciprocal per side
-// instead of seven divisions (the sum of the weights is positive, at least
-// (12 eps)^4 / 16, and finite).  Results agree with the reference form to
-// rounding.
-__device__ __forceinline__ double weno5_side(double f1, double f2, double f3, double f4, double f5) {
-  const double d1 = 1 / 16., d2 = 10 / 16., d3 = 5 / 16., eps12 = 12. * 1.e-6;
-  double t, s;
-  t = f3 - 2 * f2 + f1; s = 3. * f3 - 4. * f2 + f1;
-  double q1 = 13. * (t * t) + 3. * (s * s) + eps12;
-  t = f4 - 2 * f3 + f2; s = f4 - f2;
-  double q2 = 13. * (t * t) + 3. * (s * s) + eps12;
-  t = f5 - 2 * f4 + f3; s = f5 - 4. * f4 + 3. * f3;
-  double q3 = 13. * (t * t) + 3. * (s * s) + eps12;
-  double Q1 = q1 * q1, Q2 = q2 * q2, Q3 = q3 * q3;
-  double w1 = d1 * (Q2 * Q3), w2 = d2 * (Q1 * Q3), w3 = d3 * (Q1 * Q2);
-  double p1 = 3 / 8. * f1 + -10 / 8. * f2 + 15 / 8. * f3;
-  double p2 = -1 / 8. * f2 + 6 / 8. * f3 + 3 / 8. * f4;
-  double p3 = 3 / 8. * f3 + 6 / 8. * f4 + -1 / 8. * f5;
-  return (w1 * p1 + w2 * p2 + w3 * p3) * rcp_nr(w1 + w2 + w3);
+// WENO5 (holib.f90:177-232).  The three smoothness indicators belong to the
+// cell: its two faces use the same three numbers in opposite order, so taking
+// both faces of a cell together halves that work (per variable 57 FP64
+// instructions instead of 94 for the two sides of an interface).  With the
+// first differences d, the second differences t_j and the third differences
+// e, and Q_j = (13 t_j^2 + 3 s_j^2 + 12 eps)^2 (the reference's
+// (beta/12 + eps)^2 times 144, which cancels), the weights of the three
+// substencils are d_j times the product of the other two Q: one reciprocal
+// per face, of a positive and finite sum.  The weighted mean of the three
+// parabolas is written as the middle one plus the weighted deviations of the
+// outer two, which are third differences:  p1 - p2 = -3/8 e1,
+// p3 - p2 = -1/8 e2.
+__device__ __forceinline__ void weno5_cell(const double* f, double& hi, double& lo) {
+  const double eps12 = 12. * 1.e-6;
+  const double d0 = f[1] - f[0], d1 = f[2] - f[1], d2 = f[3] - f[2], d3 = f[4] - f[3];
+  const double t1 = d1 - d0, t2 = d2 - d1, t3 = d3 - d2;
+  const double e1 = t2 - t1, e2 = t3 - t2;
+  const double s1 = 2. * d1 + t1, s2 = d1 + d2, s3 = t3 - 2. * d2;
+  const double q1 = 3. * (s1 * s1) + (13. * (t1 * t1) + eps12);
+  const double q2 = 3. * (s2 * s2) + (13. * (t2 * t2) + eps12);
+  const double q3 = 3. * (s3 * s3) + (13. * (t3 * t3) + eps12);
+  const double Q1 = q1 * q1, Q2 = q2 * q2, Q3 = q3 * q3;
+  const double a = Q2 * Q3, b = 10. * (Q1 * Q3), c = Q1 * Q2;   // 16 x the products, without d_j of the outer ones
+  const double m1 = a * e1, m2 = c * e2;
+  const double h = (3. * m1 + 5. * m2) * rcp_nr(5. * c + (a + b));
+  const double l = (3. * m2 + 5. * m1) * rcp_nr(5. * a + (c + b));
+  hi = f[2] + 0.125 * ((3. * d2 + d1) - h);
+  lo = f[2] - 0.125 * ((3. * d1 + d2) - l);
 }
 
 __device__ __forceinline__ double weno3_side(double f1, double f2, double f3) {
@@ -353,35 +358,30 @@ __device__ __forceinline__ double ceno3_side(double f1, double f2, double f3, do
 }
 
 template <int REC>
-__device__ __forceinline__ void rec_face(const double* f, double& gl, double& gr) {
-  // f[j] = cell (i-2+j)
-  if constexpr (REC == REC_WENO5) {           // holib.f90:177-232
-    gl = weno5_side(f[0], f[1], f[2], f[3], f[4]);
-    gr = weno5_side(f[5], f[4], f[3], f[2], f[1]);
+__device__ __forceinline__ void rec_cell(const double* f, double& hi, double& lo) {
+  if constexpr (REC == REC_WENO5) {
+    weno5_cell(f, hi, lo);
   } else if constexpr (REC == REC_PPM4) {     // holib.f90:236-268
-    gl = f[2] + .5 * (f[3] - f[2]) - .125 * (mm2(f[4] - f[3], f[3] - f[2]) - mm2(f[3] - f[2], f[2] - f[1]));
-    gr = f[3] + .5 * (f[2] - f[3]) - .125 * (mm2(f[1] - f[2], f[2] - f[3]) - mm2(f[2] - f[3], f[3] - f[4]));
+    hi = f[2] + .5 * (f[3] - f[2]) - .125 * (mm2(f[4] - f[3], f[3] - f[2]) - mm2(f[3] - f[2], f[2] - f[1]));
+    lo = f[2] + .5 * (f[1] - f[2]) - .125 * (mm2(f[0] - f[1], f[1] - f[2]) - mm2(f[1] - f[2], f[2] - f[3]));
   } else if constexpr (REC == REC_TVD2) {     // holib.f90:47-77
-    gl = f[2] + .5 * mm2(f[2] - f[1], f[3] - f[2]);
-    gr = f[3] - .5 * mm2(f[3] - f[2], f[4] - f[3]);
+    const double h = .5 * mm2(f[2] - f[1], f[3] - f[2]);
+    hi = f[2] + h;
+    lo = f[2] - h;
   } else if constexpr (REC == REC_MPE5) {     // holib.f90:297-318
     const double d1 = 3 / 128., d2 = -20 / 128., d3 = 90 / 128., d4 = 60 / 128., d5 = -5 / 128.;
-    double l = d1 * f[0] + d2 * f[1] + d3 * f[2] + d4 * f[3] + d5 * f[4];
-    double r = d1 * f[5] + d2 * f[4] + d3 * f[3] + d4 * f[2] + d5 * f[1];
-    gl = mp5(l, f[0], f[1], f[2], f[3], f[4]);
-    gr = mp5(r, f[5], f[4], f[3], f[2], f[1]);
+    hi = mp5(d1 * f[0] + d2 * f[1] + d3 * f[2] + d4 * f[3] + d5 * f[4], f[0], f[1], f[2], f[3], f[4]);
+    lo = mp5(d1 * f[4] + d2 * f[3] + d3 * f[2] + d4 * f[1] + d5 * f[0], f[4], f[3], f[2], f[1], f[0]);
   } else if constexpr (REC == REC_WENO3) {    // holib.f90:130-173
-    gl = weno3_side(f[1], f[2], f[3]);
-    gr = weno3_side(f[4], f[3], f[2]);
+    hi = weno3_side(f[1], f[2], f[3]);
+    lo = weno3_side(f[3], f[2], f[1]);
   } else if constexpr (REC == REC_CENO3) {    // holib.f90:81-126
-    gl = ceno3_side(f[0], f[1], f[2], f[3], f[4]);
-    gr = ceno3_side(f[5], f[4], f[3], f[2], f[1]);
+    hi = ceno3_side(f[0], f[1], f[2], f[3], f[4]);
+    lo = ceno3_side(f[4], f[3], f[2], f[1], f[0]);
   } else {                                    // REC_MPE3, holib.f90:272-293
     const double d1 = -1 / 8., d2 = 6 / 8., d3 = 3 / 8.;
-    double l = d1 * f[1] + d2 * f[2] + d3 * f[3];
-    double r = d1 * f[4] + d2 * f[3] + d3 * f[2];
-    gl = mp5(l, f[0], f[1], f[2], f[3], f[4]);
-    gr = mp5(r, f[5], f[4], f[3], f[2], f[1]);
+    hi = mp5(d1 * f[1] + d2 * f[2] + d3 * f[3], f[0], f[1], f[2], f[3], f[4]);
+    lo = mp5(d1 * f[3] + d2 * f[2] + d3 * f[1], f[4], f[3], f[2], f[1], f[0]);
   }
 }
 
@@ -416,7 +416,7 @@ __device__ __forceinline__ PiDer derived_pi(double* p, const Metric& M) {
              g2 + vz * vx * g1 * xy * vy * g2 - vz * xx * g1 - vz * yy * g2 + vz * vx *
              vx * g1 * g1 * xx + vy * g1 * yz * vz * vz * g3 + vz * vy * g1 * g1 *
              xy * vx + vz * vy * vy * g1 * yy * g2);
-    p[KPIZZ] = (ivz * rcp_nr(g3)) * (vx * g1 * xy * vy * g2 - xx * g1 - yy * g2 +
+    p[KPIZZ] = (ivz * M.ig3) * (vx * g1 * xy * vy * g2 - xx * g1 - yy * g2 +
              vx * vx * g1 * g1 * xx + vy * g1 * yz * vz * g3 + 2. * vx * g1 * xz * vz *
              g3 + vy * g1 * g1 * xy * vx + vy * vy * g1 * yy * g2 + vz * g3 * yz *
              vy * g2);
@@ -435,7 +435,7 @@ __device__ __forceinline__ void ideal_E(const Metric& M, const double* v, double
   E[2] = -M.gp * (v[KVX] * v[KBY] - v[KVY] * v[KBX]);
 }
 __device__ __forceinline__ void e_cross_b(const Metric& M, const double* E, const double* v, double* X) {
-  double c0 = E[0], c1 = E[1], c2 = E[2] / M.g3;
+  double c0 = E[0], c1 = E[1], c2 = E[2] * M.ig3;
   X[0] = M.gp * (c1 * v[KBZ] - c2 * v[KBY]);
   X[1] = M.gp * (c2 * v[KBX] - c0 * v[KBZ]);
   X[2] = M.gp * (c0 * v[KBY] - c1 * v[KBX]);
@@ -475,7 +475,7 @@ __device__ __forceinline__ int prim2cons(const Eos& E, const Metric& M, double* 
   } else if constexpr (SysT<SYS>::MHD) {
     double Ef[3], X[3];
     ideal_E(M, v, Ef);
-    double E2 = Ef[0] * Ef[0] + Ef[1] * Ef[1] + Ef[2] * Ef[2] / M.g3;
+    double E2 = Ef[0] * Ef[0] + Ef[1] * Ef[1] + Ef[2] * Ef[2] * M.ig3;
     e_cross_b(M, Ef, v, X);
     double B2 = v[KBX] * v[KBX] + v[KBY] * v[KBY] + v[KBZ] * v[KBZ] * M.g3;
     double EEM = 0.5 * (E2 + B2);
@@ -484,7 +484,7 @@ __device__ __forceinline__ int prim2cons(const Eos& E, const Metric& M, double* 
     u[KVZ] = ww * vz * M.g3 + X[2];
     u[KPR] = ww - pr + EEM;
     u[KBX] = v[KBX]; u[KBY] = v[KBY]; u[KBZ] = v[KBZ];
-    if constexpr (SysT<SYS>::GLM) u[KGLM] = v[KGLM] / M.gp;
+    if constexpr (SysT<SYS>::GLM) u[KGLM] = v[KGLM] * M.gm;
   } else {
     u[KVX] = ww * vx;
     u[KVY] = ww * vy;
@@ -543,12 +543,12 @@ __device__ __forceinline__ int side_state(const Eos& E, const Metric& M, double*
   s.ca2 = 0.;
   if constexpr (SysT<SYS>::MHD) {
     ideal_E(M, v, s.E);
-    double E2 = s.E[0] * s.E[0] + s.E[1] * s.E[1] + s.E[2] * s.E[2] / M.g3;
+    double E2 = s.E[0] * s.E[0] + s.E[1] * s.E[1] + s.E[2] * s.E[2] * M.ig3;
     e_cross_b(M, s.E, v, s.X);
     double B2 = v[KBX] * v[KBX] + v[KBY] * v[KBY] + v[KBZ] * v[KBZ] * M.g3;
     s.EEM = 0.5 * (E2 + B2);
     double bb2 = B2 - E2;
-    s.ca2 = bb2 / (bb2 + (en + pr));
+    s.ca2 = bb2 * rcp_nr(bb2 + (en + pr));
   }
   s.vdir = DIR == 1 ? vx : (DIR == 2 ? vy : vz);
   s.wwdir = s.ww * s.vdir;
@@ -559,12 +559,12 @@ __device__ __forceinline__ int side_state(const Eos& E, const Metric& M, double*
 // fast speeds lambda+ (lp) and lambda- (lm), system.f90:1557-1580
 template <int DIR>
 __device__ __forceinline__ void side_speeds(const Metric& M, const SideState& s, double& lp, double& lm) {
-  const double gdir = DIR == 1 ? M.g1 : (DIR == 2 ? M.g2 : M.g3);
+  const double igdir = DIR == 3 ? M.ig3 : 1.;   // g1 = g2 = 1
   const double ca2 = s.ca2;
   double a2 = s.cs2 + ca2 - s.cs2 * ca2;
-  double den = 1. / (1. - s.v2 * a2);
+  double den = rcp_nr(1. - s.v2 * a2);
   double vf1 = den * (1. - a2) * s.vdir;
-  double vf2 = den * sqrt(a2 * (1. - s.v2) * ((1. - s.v2 * a2) / gdir - (1. - a2) * (s.vdir * s.vdir)));
+  double vf2 = den * sqrt(a2 * (1. - s.v2) * ((1. - s.v2 * a2) * igdir - (1. - a2) * (s.vdir * s.vdir)));
   lp = vf1 + vf2;
   lm = vf1 - vf2;
 }
@@ -580,7 +580,7 @@ __device__ __forceinline__ double u_comp(int k, const Metric& M, const SideState
       case KVY: return s.ww * v[KVY] + s.X[1];
       case KVZ: return s.ww * v[KVZ] * M.g3 + s.X[2];
       case KPR: return s.ww - s.pr + s.EEM;
-      case KGLM: return v[KGLM] / M.gp;
+      case KGLM: return v[KGLM] * M.gm;
       default: return v[k];   // B
     }
   }
@@ -613,7 +613,7 @@ __device__ __forceinline__ double f_comp(int k, const Metric& M, const SideState
         case KBX: return GLM ? v[KGLM] : 0.;
         case KBY: return -E[2] * M.gm;
         case KBZ: return +E[1] * M.gm;
-        default: return v[KBX] / M.gp;
+        default: return v[KBX] * M.gm;
       }
     } else if constexpr (DIR == 2) {
       switch (k) {
@@ -624,18 +624,18 @@ __device__ __forceinline__ double f_comp(int k, const Metric& M, const SideState
         case KBX: return E[2] * M.gm;
         case KBY: return GLM ? v[KGLM] : 0.;
         case KBZ: return -E[0] * M.gm;
-        default: return v[KBY] / M.gp;
+        default: return v[KBY] * M.gm;
       }
     } else {
       switch (k) {
-        case KVX: return wd * v[KVX] - E[2] / M.g3 * E[0] - Bz * Bx;
-        case KVY: return wd * v[KVY] - E[2] / M.g3 * E[1] - Bz * By;
-        case KVZ: return wd * v[KVZ] * M.g3 - E[2] * E[2] / M.g3 - Bz * Bz * M.g3 + s.pr + s.EEM;
-        case KPR: return wd + s.X[2] / M.g3;
+        case KVX: return wd * v[KVX] - E[2] * M.ig3 * E[0] - Bz * Bx;
+        case KVY: return wd * v[KVY] - E[2] * M.ig3 * E[1] - Bz * By;
+        case KVZ: return wd * v[KVZ] * M.g3 - E[2] * E[2] * M.ig3 - Bz * Bz * M.g3 + s.pr + s.EEM;
+        case KPR: return wd + s.X[2] * M.ig3;
         case KBX: return -E[1] * M.gm;
         case KBY: return E[0] * M.gm;
-        case KBZ: return GLM ? v[KGLM] / M.g3 : 0.;
-        default: return v[KBZ] / M.gp;
+        case KBZ: return GLM ? v[KGLM] * M.ig3 : 0.;
+        default: return v[KBZ] * M.gm;
       }
     }
   }
@@ -1082,7 +1082,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
   double d = gm * u[KRH];
   double sx = gm * u[KVX];
   double sy = gm * u[KVY];
-  double sz = gm * u[KVZ] / M.g3;
+  double sz = gm * u[KVZ] * M.ig3;
   double et = gm * u[KPR];
   double s2 = M.g1 * sx * sx + M.g2 * sy * sy + M.g3 * sz * sz;
   // eos_pressure leaves its outputs unset on an error (out of table range)
@@ -1133,7 +1133,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
       double sz_cov = uin[KVZ] - q.pitz * M.g3;
       sx = sx_cov;
       sy = sy_cov;
-      sz = sz_cov / M.g3;
+      sz = sz_cov * M.ig3;
       s2 = sx * sx_cov + sy * sy_cov + sz * sz_cov;
       pr = v[KPR];
       for (int ip = 1; ip <= 100; ip++) {
@@ -1201,7 +1201,7 @@ __device__ __forceinline__ EmTerms em_terms(const Metric& M, const double* Ev, c
 __device__ __forceinline__ void cross_contra(const Metric& M, const double* a, const double* b, double* c) {
   c[0] = M.gp * (a[1] * b[2] - a[2] * b[1]);
   c[1] = M.gp * (a[2] * b[0] - a[0] * b[2]);
-  c[2] = M.gp * (a[0] * b[1] - a[1] * b[0]) / M.g3;
+  c[2] = M.gp * (a[0] * b[1] - a[1] * b[0]) * M.ig3;
 }
 
 template <int SYS, bool ZZ>
@@ -1244,7 +1244,7 @@ __device__ int res_side_state(const Eos& E, const Metric& M, double* v, SideStat
   }
   s.EEM = t.eem;
   const double bb2 = dmax(t.B2 - t.E2, 0.);
-  s.ca2 = bb2 / (bb2 + s.enpr);
+  s.ca2 = bb2 * rcp_nr(bb2 + s.enpr);
   return 0;
 }
 
@@ -1259,7 +1259,7 @@ __device__ double res_u_comp(int k, const Metric& M, const SideState& s, const d
     else if (k == KPR) r = r + s.EEM;
     return r;
   }
-  if (k == T::KG) return v[T::KG] / M.gp;
+  if (k == T::KG) return v[T::KG] * M.gm;
   return v[k];   // B, E
 }
 
@@ -1277,7 +1277,7 @@ __device__ double res_f_comp(int k, const Metric& M, const SideState& s, const d
     if (k == KVX) em = -Ev[D] * Ec[0] - B[D] * B[0] + (D == 0 ? s.EEM : 0.);
     else if (k == KVY) em = -Ev[D] * Ec[1] - B[D] * B[1] + (D == 1 ? s.EEM : 0.);
     else if (k == KVZ) em = -Ev[D] * Ec[2] - B[D] * B[2] * M.g3 + (D == 2 ? s.EEM : 0.);
-    else if (k == KPR) em = D == 2 ? s.X[2] / M.g3 : s.X[D];
+    else if (k == KPR) em = D == 2 ? s.X[2] * M.ig3 : s.X[D];
     else return r;
     return r + em;
   }
@@ -1289,7 +1289,7 @@ __device__ double res_f_comp(int k, const Metric& M, const SideState& s, const d
     if (k == T::KE) return 0.;
     if (k == T::KE + 1) return B[2] * M.g3 * M.gm;
     if (k == T::KE + 2) return -B[1] * M.g2 * M.gm;
-    return B[0] / M.gp;
+    return B[0] * M.gm;
   } else if constexpr (DIR == 2) {
     if (k == T::KB) return Ec[2] * M.gm;
     if (k == T::KB + 1) return psi;
@@ -1297,15 +1297,15 @@ __device__ double res_f_comp(int k, const Metric& M, const SideState& s, const d
     if (k == T::KE) return -B[2] * M.g3 * M.gm;
     if (k == T::KE + 1) return 0.;
     if (k == T::KE + 2) return B[0] * M.g1 * M.gm;
-    return B[1] / M.gp;
+    return B[1] * M.gm;
   } else {
     if (k == T::KB) return -Ec[1] * M.gm;
     if (k == T::KB + 1) return Ec[0] * M.gm;
-    if (k == T::KB + 2) return psi / M.g3;
+    if (k == T::KB + 2) return psi * M.ig3;
     if (k == T::KE) return B[1] * M.g2 * M.gm;
     if (k == T::KE + 1) return -B[0] * M.g1 * M.gm;
     if (k == T::KE + 2) return 0.;
-    return B[2] / M.gp;
+    return B[2] * M.gm;
   }
 }
 

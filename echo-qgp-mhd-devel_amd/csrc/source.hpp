@@ -140,12 +140,12 @@ __device__ __forceinline__ int sys_source(const Eos& E, const Metric& M, int coo
         double Ef[3];
         ideal_E(M, v, Ef);
         double B2 = v[KBX] * v[KBX] + v[KBY] * v[KBY] + v[KBZ] * v[KBZ] * M.g3;
-        double E2 = Ef[0] * Ef[0] + Ef[1] * Ef[1] + Ef[2] * Ef[2] / M.g3;
+        double E2 = Ef[0] * Ef[0] + Ef[1] * Ef[1] + Ef[2] * Ef[2] * M.ig3;
         double EEM = 0.5 * (E2 + B2);
-        double e3 = Ef[2] / M.g3;
-        src[KPR] = -t * (ww * vz * vz - e3 * e3 - v[KBZ] * v[KBZ] + (EEM + pr) / M.g3);
+        double e3 = Ef[2] * M.ig3;
+        src[KPR] = -t * (ww * vz * vz - e3 * e3 - v[KBZ] * v[KBZ] + (EEM + pr) * M.ig3);
       } else {
-        src[KPR] = -t * (ww * vz * vz + pr / M.g3);
+        src[KPR] = -t * (ww * vz * vz + pr * M.ig3);
       }
     }
   } else {
@@ -264,7 +264,7 @@ __device__ __forceinline__ int res_source(const Eos& E, const Metric& M, int coo
   const double vel[3] = {v[KVX], v[KVY], v[KVZ]};
   if (coordinates == BJORKEN) {
     const EmTerms t = em_terms(M, Ev, B);
-    src[KPR] = src[KPR] + (-M.t * (t.eem / M.g3 - Ev[2] * Ev[2] - B[2] * B[2])) * M.gp;
+    src[KPR] = src[KPR] + (-M.t * (t.eem * M.ig3 - Ev[2] * Ev[2] - B[2] * B[2])) * M.gp;
   }
   double S[3];
   ohm_stiff(M, vel, Ev, B, sig, sch, S);
