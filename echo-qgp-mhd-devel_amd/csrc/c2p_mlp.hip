@@ -297,8 +297,10 @@ int echo_cons2prim_batch_dev(echo_grid* g, const double* d_u, double* d_v, int32
   HIPCHECK(hipSetDevice(g->dev));
   if (g->timing) HIPCHECK(hipEventRecord(g->ev[0], g->stream));
   dispatch_sys(g->cfg, [&](auto sys, auto zz) {
-    k_c2p_batch<decltype(sys)::value, decltype(zz)::value>
-        <<<nblocks(n, UPDATE_BLOCK), UPDATE_BLOCK, 0, g->stream>>>(g->ga, d_u, d_v, d_status, n);
+    dispatch_algo<decltype(sys)::value>(g->cfg, [&](auto algo) {
+      k_c2p_batch<decltype(sys)::value, decltype(zz)::value, decltype(algo)::value>
+          <<<nblocks(n, UPDATE_BLOCK), UPDATE_BLOCK, 0, g->stream>>>(g->ga, d_u, d_v, d_status, n);
+    });
   });
   HIPCHECK(hipGetLastError());
   if (g->timing) HIPCHECK(hipEventRecord(g->ev[1], g->stream));

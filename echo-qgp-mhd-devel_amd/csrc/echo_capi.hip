@@ -93,9 +93,11 @@ static void enqueue_stage_t(echo_grid* g, int irk) {
   const bool last = (irk == nrk);
   double* Ucur = (irk == 1) ? g->U[0] : g->U[1];
   double* Uout = last ? g->U[0] : g->U[1];
-  k_update<SYS, ZZ><<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(
-      g->ga, g->V, g->U[0], Ucur, Uout, g->F[0], g->F[1], g->F[2], g->L[0], g->L[1], g->L[2],
-      g->VS[0], g->VS[1], g->fix, c1, c2, irk == 1 ? 1 : 0, last ? 1 : 0);
+  dispatch_algo<SYS>(g->cfg, [&](auto algo) {
+    k_update<SYS, ZZ, decltype(algo)::value><<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(
+        g->ga, g->V, g->U[0], Ucur, Uout, g->F[0], g->F[1], g->F[2], g->L[0], g->L[1], g->L[2],
+        g->VS[0], g->VS[1], g->fix, c1, c2, irk == 1 ? 1 : 0, last ? 1 : 0);
+  });
   if (g->net) enqueue_net_c2p(g, Uout);   // ideal MHD with the learned inversion
   if (g->timing) hipEventRecord(g->ev[5], g->stream);
   // con2prim repair of the cells k_update could not invert (rare; returns at
@@ -942,8 +944,10 @@ int echo_cons2prim_batch(echo_grid* g, const double* u, double* v, int32_t* stat
   HIPCHECK(hipMemcpyAsync(dv, v, sz, hipMemcpyHostToDevice, g->stream));
   dim3 grid(nblocks(n, UPDATE_BLOCK));
   dispatch_sys(g->cfg, [&](auto sys, auto zz) {
-    k_c2p_batch<decltype(sys)::value, decltype(zz)::value>
-        <<<grid, UPDATE_BLOCK, 0, g->stream>>>(g->ga, du, dv, ds, n);
+    dispatch_algo<decltype(sys)::value>(g->cfg, [&](auto algo) {
+      k_c2p_batch<decltype(sys)::value, decltype(zz)::value, decltype(algo)::value>
+          <<<grid, UPDATE_BLOCK, 0, g->stream>>>(g->ga, du, dv, ds, n);
+    });
   });
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipMemcpyAsync(v, dv, sz, hipMemcpyDeviceToHost, g->stream));

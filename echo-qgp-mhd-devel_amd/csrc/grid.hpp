@@ -153,6 +153,16 @@ inline void dispatch_sys(const echo_config& c, Fn&& fn) {
   }
 }
 
+// the ideal-MHD inversion algorithm as a compile-time constant for the kernels
+// that take it (ALGO): 5, or 0 for the rest
+template <int SYS, typename Fn>
+inline void dispatch_algo(const echo_config& c, Fn&& fn) {
+  if constexpr (SysT<SYS>::MHD) {
+    if (c.algo_solver == 5) return fn(std::integral_constant<int, 5>());
+  }
+  fn(std::integral_constant<int, 0>());
+}
+
 // find_pressure_from_temperature (eos.f90:1221-1252) on a host copy of the
 // EoS, with the lower bisection bound started at 0 (the reference leaves it
 // uninitialised); the bisection stops at |T(p) - T| <= 1e-10 T

@@ -128,24 +128,24 @@ __device__ __forceinline__ long long xcd_block(unsigned b, unsigned nb) {
 constexpr int UPD_TX = 64, UPD_TZ = 4;
 static_assert(UPDATE_BLOCK == UPD_TX * UPD_TZ && UPD_TX == 64, "a tile row is one wave of 64 lanes");
 __device__ __forceinline__ bool update_cell(const GridArgs& a, int& x, int& y, int& z, long long& c) {
-  const long long b = xcd_block(blockIdx.x, gridDim.x);
+  // (a grid that fits in memory has fewer than 2^32 cells)
+  const unsigned b = (unsigned)xcd_block(blockIdx.x, gridDim.x), nx = (unsigned)a.nx, ny = (unsigned)a.ny;
   if (a.upd_tz == 1) {
-    c = b * UPDATE_BLOCK + threadIdx.x;
+    c = (long long)b * UPDATE_BLOCK + threadIdx.x;
     if (c >= a.N) return false;
-    x = (int)(c % a.nx);
-    const long long r = c / a.nx;
-    y = (int)(r % a.ny);
-    z = (int)(r / a.ny);
+    const unsigned i = (unsigned)c, r = i / nx;
+    x = (int)(i - r * nx);
+    z = (int)(r / ny);
+    y = (int)(r - (unsigned)z * ny);
     return true;
   }
-  const int nxc = (a.nx + UPD_TX - 1) / UPD_TX;
-  const long long r = b / nxc;
-  x = (int)(b % nxc) * UPD_TX + (int)(threadIdx.x & (UPD_TX - 1));
-  y = (int)(r % a.ny);
-  const long long zz = (r / a.ny) * UPD_TZ + (threadIdx.x >> 6);
-  if (x >= a.nx || zz >= a.nz) return false;
-  z = (int)zz;
-  c = x + (long long)a.nx * (y + (long long)a.ny * z);
+  const unsigned nxc = (nx + UPD_TX - 1) / UPD_TX;
+  const unsigned r = b / nxc, rz = r / ny;
+  x = (int)((b - r * nxc) * UPD_TX + (threadIdx.x & (UPD_TX - 1)));
+  y = (int)(r - rz * ny);
+  z = (int)(rz * UPD_TZ + (threadIdx.x >> 6));
+  if (x >= a.nx || z >= a.nz) return false;
+  c = x + (long long)nx * (y + ny * (unsigned)z);
   return true;
 }
 
@@ -613,19 +613,19 @@ __device__ __forceinline__ Deriv cell_deriv(const GridArgs& a, const Metric& M, 
   double dx[4] = {0., 0., 0., 0.}, dy[4] = {0., 0., 0., 0.}, dz[4] = {0., 0., 0., 0.};
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   if (nx > 1) {
-    long long nf = (long long)(nx + 1) * ny * nz, f0 = x + (long long)(nx + 1) * (y + (long long)ny * z);
+    const unsigned nf = (unsigned)(nx + 1) * ny * nz, f0 = x + (unsigned)(nx + 1) * (y + (unsigned)ny * z);
 #pragma unroll
-    for (int q = 0; q < 4; q++) dx[q] = a.ddx * 0.5 * (LX[q * nf + f0 + 1] - LX[q * nf + f0]);
+    for (int q = 0; q < 4; q++) dx[q] = a.ddx * 0.5 * (LX[(long long)q * nf + f0 + 1] - LX[(long long)q * nf + f0]);
   }
   if (ny > 1) {
-    long long nf = (long long)nx * (ny + 1) * nz, f0 = x + (long long)nx * (y + (long long)(ny + 1) * z);
+    const unsigned nf = (unsigned)nx * (ny + 1) * nz, f0 = x + (unsigned)nx * (y + (unsigned)(ny + 1) * z);
 #pragma unroll
-    for (int q = 0; q < 4; q++) dy[q] = a.ddy * 0.5 * (LY[q * nf + f0 + nx] - LY[q * nf + f0]);
+    for (int q = 0; q < 4; q++) dy[q] = a.ddy * 0.5 * (LY[(long long)q * nf + f0 + nx] - LY[(long long)q * nf + f0]);
   }
   if (nz > 1) {
-    long long nf = (long long)nx * ny * (nz + 1), f0 = x + (long long)nx * (y + (long long)ny * z);
+    const unsigned nf = (unsigned)nx * ny * (nz + 1), f0 = x + (unsigned)nx * (y + (unsigned)ny * z);
 #pragma unroll
-    for (int q = 0; q < 4; q++) dz[q] = a.ddz * 0.5 * (LZ[q * nf + f0 + (long long)nx * ny] - LZ[q * nf + f0]);
+    for (int q = 0; q < 4; q++) dz[q] = a.ddz * 0.5 * (LZ[(long long)q * nf + f0 + (unsigned)nx * ny] - LZ[(long long)q * nf + f0]);
   }
   D.dutdx = dx[0]; D.duxdx = dx[1]; D.duydx = dx[2]; D.duzdx = dx[3];
   D.dutdy = dy[0]; D.duxdy = dy[1]; D.duydy = dy[2]; D.duzdy = dy[3];
@@ -638,12 +638,13 @@ __device__ __forceinline__ Deriv cell_deriv(const GridArgs& a, const Metric& M, 
     const long long N = a.N;
     double ox = VSo[c], oy = VSo[N + c], oz = VSo[2 * N + c];
     double nxv = VSn[c], nyv = VSn[N + c], nzv = VSn[2 * N + c];
-    double gamma1 = 1. / sqrt(1. - M.g1 * (ox * ox) - M.g2 * (oy * oy) - S->g_cov_3_old * (oz * oz));
-    double gamma2 = 1. / sqrt(1. - M.g1 * (nxv * nxv) - M.g2 * (nyv * nyv) - M.g3 * (nzv * nzv));
-    D.dutdt = (gamma2 - gamma1) / ti;
-    D.duxdt = (gamma2 * nxv - gamma1 * ox) / ti;
-    D.duydt = (gamma2 * nyv - gamma1 * oy) / ti;
-    D.duzdt = (gamma2 * nzv - gamma1 * oz) / ti;
+    const double gamma1 = rsqrt_nr(1. - M.g1 * (ox * ox) - M.g2 * (oy * oy) - S->g_cov_3_old * (oz * oz));
+    const double gamma2 = rsqrt_nr(1. - M.g1 * (nxv * nxv) - M.g2 * (nyv * nyv) - M.g3 * (nzv * nzv));
+    const double iti = 1. / ti;
+    D.dutdt = (gamma2 - gamma1) * iti;
+    D.duxdt = (gamma2 * nxv - gamma1 * ox) * iti;
+    D.duydt = (gamma2 * nyv - gamma1 * oy) * iti;
+    D.duzdt = (gamma2 * nzv - gamma1 * oz) * iti;
   }
   return D;
 }
@@ -658,16 +659,16 @@ __device__ __forceinline__ double res_div_e(const GridArgs& a, int x, int y, int
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   double r = 0.;
   if (nx > 1) {
-    const long long nf = (long long)(nx + 1) * ny * nz, f0 = x + (long long)(nx + 1) * (y + (long long)ny * z);
-    r = r + (FX[nv * nf + f0] + FX[nv * nf + f0 + 1]) * (a.ddx / 2.);
+    const unsigned nf = (unsigned)(nx + 1) * ny * nz, f0 = x + (unsigned)(nx + 1) * (y + (unsigned)ny * z);
+    r = r + (FX[(long long)nv * nf + f0] + FX[(long long)nv * nf + f0 + 1]) * (a.ddx / 2.);
   }
   if (ny > 1) {
-    const long long nf = (long long)nx * (ny + 1) * nz, f0 = x + (long long)nx * (y + (long long)(ny + 1) * z);
-    r = r + (FY[nv * nf + f0] + FY[nv * nf + f0 + nx]) * (a.ddy / 2.);
+    const unsigned nf = (unsigned)nx * (ny + 1) * nz, f0 = x + (unsigned)nx * (y + (unsigned)(ny + 1) * z);
+    r = r + (FY[(long long)nv * nf + f0] + FY[(long long)nv * nf + f0 + nx]) * (a.ddy / 2.);
   }
   if (nz > 1) {
-    const long long nf = (long long)nx * ny * (nz + 1), f0 = x + (long long)nx * (y + (long long)ny * z);
-    r = r + (FZ[nv * nf + f0] + FZ[nv * nf + f0 + (long long)nx * ny]) * (a.ddz / 2.);
+    const unsigned nf = (unsigned)nx * ny * (nz + 1), f0 = x + (unsigned)nx * (y + (unsigned)ny * z);
+    r = r + (FZ[(long long)nv * nf + f0] + FZ[(long long)nv * nf + f0 + (unsigned)nx * ny]) * (a.ddz / 2.);
   }
   return r;
 }
@@ -682,22 +683,34 @@ __device__ __forceinline__ void flux_div(const GridArgs& a, int x, int y, int z,
 #pragma unroll
   for (int k = 0; k < NV; k++) du[k] = 0.;
   if (nx > 1) {
-    long long nf = (long long)(nx + 1) * ny * nz, f0 = x + (long long)(nx + 1) * (y + (long long)ny * z);
+    const unsigned nf = (unsigned)(nx + 1) * ny * nz, f0 = x + (unsigned)(nx + 1) * (y + (unsigned)ny * z);
 #pragma unroll
-    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddx * (FX[k * nf + f0 + 1] - FX[k * nf + f0]);
+    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddx * (FX[(long long)k * nf + f0 + 1] - FX[(long long)k * nf + f0]);
   }
   if (ny > 1) {
-    long long nf = (long long)nx * (ny + 1) * nz, f0 = x + (long long)nx * (y + (long long)(ny + 1) * z);
+    const unsigned nf = (unsigned)nx * (ny + 1) * nz, f0 = x + (unsigned)nx * (y + (unsigned)(ny + 1) * z);
 #pragma unroll
-    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddy * (FY[k * nf + f0 + nx] - FY[k * nf + f0]);
+    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddy * (FY[(long long)k * nf + f0 + nx] - FY[(long long)k * nf + f0]);
   }
   if (nz > 1) {
-    long long nf = (long long)nx * ny * (nz + 1), f0 = x + (long long)nx * (y + (long long)ny * z);
-    const long long st = (long long)nx * ny;
+    const unsigned nf = (unsigned)nx * ny * (nz + 1), f0 = x + (unsigned)nx * (y + (unsigned)ny * z);
+    const unsigned st = (unsigned)nx * ny;
 #pragma unroll
-    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddz * (FZ[k * nf + f0 + st] - FZ[k * nf + f0]);
+    for (int k = 0; k < NV; k++) du[k] = du[k] + a.ddz * (FZ[(long long)k * nf + f0 + st] - FZ[(long long)k * nf + f0]);
   }
 }
+
+// Waves per SIMD that the update's registers allow for (192 x 192 x 128
+// cells).  Three (168 VGPRs) for viscous hydro and ideal MHD, without
+// spills: ideal MHD 0.195 ms instead of 0.208 at two on 160 x 150 x 70 cells,
+// viscous hydro the same at both; at four both spill (viscous hydro 1.29
+// instead of 0.93 ms).  The viscous resistive RK update spills 164 bytes at
+// three (0.524 instead of 0.483 ms on 131 x 117 x 75 cells); its IMEX stages
+// 2 and 3 only 60, which pays (1.48 instead of 1.52 ms a launch).
+template <int SYS>
+constexpr int update_waves() { return SYS == SYS_VRMHD ? 2 : SysT<SYS>::NV > 5 ? 3 : 4; }
+template <int SYS, int STAGE>
+constexpr int imex_update_waves() { return SYS == SYS_VRMHD ? (STAGE == 4 ? 2 : 3) : 1; }
 
 // ---------------------------------------------------------------------------
 // k_update: one thread per cell.  Flux divergence (evolve.f90:383 and the
@@ -709,8 +722,14 @@ __device__ __forceinline__ void flux_div(const GridArgs& a, int x, int y, int z,
 // reads of the other cells is kept in fb: every cell's pressure before the
 // stage, and u before the smoothing of the smoothed cells.
 // ---------------------------------------------------------------------------
-template <int SYS, bool ZZ>
-__global__ __launch_bounds__(UPDATE_BLOCK) void k_update(
+//
+// ALGO: the ideal-MHD inversion algorithm when the launch knows it (5), else 0
+// (read from the arguments).  With all algorithms in one kernel the ideal-MHD
+// update needs 178 VGPRs, two waves per SIMD; with algorithm 5 alone it runs
+// three without spills (0.195 instead of 0.288 ms a launch on 160 x 150 x 70
+// cells, with the divisions taken out of algorithm 5).
+template <int SYS, bool ZZ, int ALGO>
+__global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
     GridArgs a, double* __restrict__ V, double* U0, const double* Ucur, double* Uout,
     const double* __restrict__ FX, const double* __restrict__ FY, const double* __restrict__ FZ,
     const double* __restrict__ LX, const double* __restrict__ LY, const double* __restrict__ LZ,
@@ -799,7 +818,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_update(
       return;
     }
   }
-  int e = cons2prim<SYS, ZZ>(a.eos, M, un, v, a.algo_solver);
+  int e = cons2prim<SYS, ZZ>(a.eos, M, un, v, ALGO ? ALGO : a.algo_solver);
   if (e != 0) {
     atomicOr(&fb.failbits[c >> 5], 1u << (c & 31));
     atomicAdd(&S->nfail, 1);
@@ -973,7 +992,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_imex_u2v(GridArgs a, double* _
 // result with the GLM damping of psi (evolve.f90:262), its plain inversion
 // and the viscous smoothing (STAGE 4)
 template <int SYS, bool ZZ, int STAGE>
-__global__ __launch_bounds__(UPDATE_BLOCK) void k_update_imex(
+__global__ __launch_bounds__(UPDATE_BLOCK, (imex_update_waves<SYS, STAGE>())) void k_update_imex(
     GridArgs a, double* __restrict__ V, double* __restrict__ U0, double* __restrict__ Ust,
     const double* __restrict__ FX, const double* __restrict__ FY, const double* __restrict__ FZ,
     const double* __restrict__ LX, const double* __restrict__ LY, const double* __restrict__ LZ,
@@ -1708,8 +1727,9 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_glauber_bfield(GridArgs a, BFi
   V[(KB + 2) * N + c] = bz;
 }
 
-// batched con2prim over n independent states (system_cons2prim)
-template <int SYS, bool ZZ>
+// batched con2prim over n independent states (system_cons2prim); ALGO as in
+// k_update
+template <int SYS, bool ZZ, int ALGO>
 __global__ __launch_bounds__(UPDATE_BLOCK) void k_c2p_batch(GridArgs a, const double* __restrict__ Ub,
                                                             double* __restrict__ Vb,
                                                             int* __restrict__ status, long long n) {
@@ -1720,7 +1740,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_c2p_batch(GridArgs a, const do
   double u[NV], v[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) { u[k] = Ub[k * n + i]; v[k] = Vb[k * n + i]; }
-  status[i] = cons2prim<SYS, ZZ>(a.eos, M, u, v, a.algo_solver);
+  status[i] = cons2prim<SYS, ZZ>(a.eos, M, u, v, ALGO ? ALGO : a.algo_solver);
 #pragma unroll
   for (int k = 0; k < NV; k++) Vb[k * n + i] = v[k];
 }

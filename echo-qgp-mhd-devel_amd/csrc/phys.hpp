@@ -76,6 +76,37 @@ __host__ __device__ __forceinline__ Metric make_metric(int coordinates, double t
 __host__ __device__ __forceinline__ double dmin(double a, double b) { return a < b ? a : b; }
 __host__ __device__ __forceinline__ double dmax(double a, double b) { return a > b ? a : b; }
 
+// 1/x for finite x != 0 in the normal range: the hardware reciprocal (relative
+// error e below 2^-22) and one cubic step r (1 + e + e^2), whose error e^3 is
+// below the rounding, in four instructions instead of the ten of the IEEE
+// division sequence.
+__device__ __forceinline__ double rcp_nr(double x) {
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+
+// 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
+// hardware reciprocal square root and one cubic step r (1 + e/2 + 3 e^2/8),
+// e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
+__device__ __forceinline__ double rsqrt_nr(double x) {
+  const double r = __builtin_amdgcn_rsq(x);
+  const double e = __builtin_fma(-(x * r), r, 1.0);
+  const double y = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
+  return x == 0.0 ? __builtin_inf() : y;
+}
+
+// x / d for finite d != 0 in the normal range, by the reciprocal on the device
+// (four instructions and a product instead of the IEEE sequence; within about
+// an ulp of the quotient)
+__host__ __device__ __forceinline__ double quot(double x, double d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return x * rcp_nr(d);
+#else
+  return x / d;
+#endif
+}
+
 // ---------------------------------------------------------------------------
 // Equation of state (eos.f90, numerically = 0)
 // ---------------------------------------------------------------------------
@@ -150,12 +181,10 @@ __host__ __device__ __forceinline__ int eos_pressure(const Eos& E, double rh, do
   if (en > E.te[E.n - 1]) return 124;
   int l = bracket_e(E, en);
   double p2 = E.tp[l], p1 = E.tp[l - 1], e2 = E.te[l], e1 = E.te[l - 1];
-  double t2 = E.tt[l], t1 = E.tt[l - 1];
-  pr = p1 + (p2 - p1) * (en - e1) / (e2 - e1);
-  double dpdt = (p2 - p1) / (t2 - t1);
-  double dedt = (e2 - e1) / (t2 - t1);
+  // the reference's dp/de = (dp/dT) / (de/dT) is the bracket's slope
+  dprden = quot(p2 - p1, e2 - e1);
+  pr = p1 + dprden * (en - e1);
   dprdrh = 0;
-  dprden = dpdt / dedt;
   return 0;
 }
 
@@ -170,7 +199,7 @@ __host__ __device__ __forceinline__ int eos_energy(const Eos& E, double rh, doub
   if (pr > E.tp[E.n - 1]) return 126;
   int l = bracket_p(E, pr);
   double p2 = E.tp[l], p1 = E.tp[l - 1], e2 = E.te[l], e1 = E.te[l - 1];
-  en = e1 + (e2 - e1) * (pr - p1) / (p2 - p1);
+  en = e1 + quot((e2 - e1) * (pr - p1), p2 - p1);
   return 0;
 }
 
@@ -188,7 +217,7 @@ __host__ __device__ __forceinline__ int eos_sound(const Eos& E, double rh, doubl
   if (en > E.te[E.n - 1]) return 132;
   int l = bracket_e(E, en);
   double s2 = E.tc[l], s1 = E.tc[l - 1], e2 = E.te[l], e1 = E.te[l - 1];
-  cs2 = s1 + (s2 - s1) * (en - e1) / (e2 - e1);
+  cs2 = s1 + quot((s2 - s1) * (en - e1), e2 - e1);
   return 0;
 }
 
@@ -211,12 +240,12 @@ __host__ __device__ __forceinline__ int eos_energy_sound(const Eos& E, double rh
   if (pr > E.tp[E.n - 1]) return 126;
   const int l = bracket_p(E, pr);
   const double p2 = E.tp[l], p1 = E.tp[l - 1], e2 = E.te[l], e1 = E.te[l - 1];
-  en = e1 + (e2 - e1) * (pr - p1) / (p2 - p1);
+  en = e1 + quot((e2 - e1) * (pr - p1), p2 - p1);
   if (en < E.te[0]) { err_sound = 131; return 0; }
   if (en > E.te[E.n - 1]) { err_sound = 132; return 0; }
   const int m = (en > e1 && en < e2) ? l : bracket_e(E, en);
   const double s2 = E.tc[m], s1 = E.tc[m - 1], f2 = E.te[m], f1 = E.te[m - 1];
-  cs2 = s1 + (s2 - s1) * (en - f1) / (f2 - f1);
+  cs2 = s1 + quot((s2 - s1) * (en - f1), f2 - f1);
   return 0;
 }
 
@@ -239,26 +268,6 @@ __host__ __device__ __forceinline__ int get_derived_data(const Eos& E, double rh
   en = e1 + (e2 - e1) * f;
   s = (en + pr) / temp;
   return 0;
-}
-
-// 1/x for finite x > 0 in the normal range: the hardware reciprocal (relative
-// error e below 2^-22) and one cubic step r (1 + e + e^2), whose error e^3 is
-// below the rounding, in four instructions instead of the ten of the IEEE
-// division sequence.
-__device__ __forceinline__ double rcp_nr(double x) {
-  const double r = __builtin_amdgcn_rcp(x);
-  const double e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, __builtin_fma(e, e, e), r);
-}
-
-// 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
-// hardware reciprocal square root and one cubic step r (1 + e/2 + 3 e^2/8),
-// e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
-__device__ __forceinline__ double rsqrt_nr(double x) {
-  const double r = __builtin_amdgcn_rsq(x);
-  const double e = __builtin_fma(-(x * r), r, 1.0);
-  const double y = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
-  return x == 0.0 ? __builtin_inf() : y;
 }
 
 // ---------------------------------------------------------------------------
@@ -453,7 +462,7 @@ __device__ __forceinline__ int prim2cons(const Eos& E, const Metric& M, double* 
   int err = eos_energy(E, rh, pr, en);
   if (err > 0) return err;
   double v2 = M.g1 * vx * vx + M.g2 * vy * vy + M.g3 * vz * vz;
-  double glf = 1. / sqrt(1. - v2);
+  double glf = rsqrt_nr(1. - v2);
   double w = en + pr;
   double ww = w * (glf * glf);
   u[KRH] = rh * glf;
@@ -675,33 +684,43 @@ __device__ __forceinline__ double f_comp(int k, const Metric& M, const SideState
 // ---------------------------------------------------------------------------
 struct MhdPar { double B2, SB2, S2, UU, D; };
 
+// x^(1/3) for x > 0, the start of the cubic's Newton iteration: the hardware's
+// single-precision logarithm and power (1e-6) and one Newton step on r^3 = x;
+// pow outside the range of a float
+__device__ __forceinline__ double cbrt_start(double x) {
+  if (!(x > 1e-30 && x < 1e30)) return pow(x, 1.0 / 3.0);
+  const double r = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)x) * (1.0f / 3.0f));
+  const double r2 = r * r;
+  return r - quot(r2 * r - x, 3. * r2);
+}
+
 template <bool IDEALGAS>
 __device__ __forceinline__ void mhd_cubic(const MhdPar& P, double x, double& f, double& df, double& wout) {
-  const double third = 1.0 / 3.0;
   const double gam = IDEALGAS ? (GAMMA_AD - 1) / GAMMA_AD : 0.25;
   double v2 = x;
   double rho = IDEALGAS ? P.D * sqrt(1.0 - v2) : 0.;
   double c3 = 1.0 - gam * (1.0 - v2);
+  const double ic3 = rcp_nr(c3);   // c3 in [0.75, 1]
   double c2 = IDEALGAS ? gam * rho + .5 * P.B2 * (1.0 + v2) - P.UU : .5 * P.B2 * (1.0 + v2) - P.UU;
   double c0 = -0.5 * P.SB2;
   double w;
   if (!IDEALGAS && c0 == 0.0) {
-    w = -c2 / c3;
+    w = -c2 * ic3;
   } else {
-    w = dmax(-c2 / c3, pow(-c0 / c3, third));
+    w = dmax(-c2 * ic3, cbrt_start(-c0 * ic3));
     const int nit = IDEALGAS ? 50 : 100;
     const double tol = IDEALGAS ? 1.e-10 : 1.e-12;
     for (int iter = 1; iter <= nit; iter++) {
-      double dw = -((c3 * w + c2) * (w * w) + c0) / ((3 * c3 * w + 2 * c2) * w);
-      if (fabs(dw / w) < tol) break;
+      double dw = -quot((c3 * w + c2) * (w * w) + c0, (3 * c3 * w + 2 * c2) * w);
+      if (fabs(dw) < tol * fabs(w)) break;
       w = w + dw;
     }
   }
   double dc3 = gam;
   double dc2 = IDEALGAS ? .5 * (P.B2 - gam * rho / (1. - v2)) : .5 * P.B2;
-  double dlogw = -(dc3 * w + dc2) / (3 * c3 * w + 2 * c2);
+  double dlogw = -quot(dc3 * w + dc2, 3 * c3 * w + 2 * c2);
   double wb = w + P.B2;
-  double vb2 = P.SB2 / (w * w);
+  double vb2 = quot(P.SB2, w * w);
   f = (wb * wb) * v2 - (2 * w + P.B2) * vb2 - P.S2;
   df = wb * (wb + 2 * dlogw * (w * v2 + vb2));
   wout = w;
@@ -721,7 +740,7 @@ __device__ __forceinline__ double mhd_rtsafe(const MhdPar& P, double x0, double 
       if (xl == r) { mhd_cubic<IDEALGAS>(P, r, f, df, w); return r; }
     } else {
       dxold = dx;
-      dx = f / df;
+      dx = quot(f, df);
       temp = r;
       r = r - dx;
       if (temp == r) { mhd_cubic<IDEALGAS>(P, r, f, df, w); return r; }
@@ -1089,28 +1108,33 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
   // and the Newton step still uses them (system.f90:534-538, 627-631);
   // before the first successful call the reference reads uninitialised
   // locals there.  They start at 0 here.
-  double pr, w = 0., v2, glf, rh = 0., en, drhdpr, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
+  double pr, w = 0., iw = 0., v2 = 0., glf, rh = 0., en, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
   if constexpr (!VISC) {
     pr = v[KPR];
     for (int iter = 1; iter <= 100; iter++) {
       w = et + pr;
-      v2 = s2 / (w * w);
-      if (v2 >= 1.) return 777;
-      glf = 1. / sqrt(1. - v2);
-      rh = d / glf;
+      iw = rcp_nr(w);
+      v2 = s2 * (iw * iw);
+      if (v2 >= 1. || (w == 0. && s2 > 0.)) return 777;
       en = w * (1. - v2) - pr;
-      drhdpr = rh * v2 * glf / (en + pr);
+      double drh = 0.;   // dp/drho drho/dp: the ideal gas only
+      if (E.eqstate == 2) {
+        glf = 1. / sqrt(1. - v2);
+        rh = d / glf;
+        drh = rh * v2 * glf / (en + pr);
+      }
       errcode = eos_pressure(E, rh, en, pr_eos, dprdrh, dprden);
       f = pr_eos - pr;
-      df = dprdrh * drhdpr + dprden * v2 - 1.;
-      dpr = -f / df;
+      df = dprdrh * drh + dprden * v2 - 1.;
+      dpr = -quot(f, df);
       if (fabs(dpr) < tol * pr) break;
       pr = pr + dpr;
     }
+    if (E.eqstate != 2) rh = d * sqrt(1. - v2);
     v[KRH] = rh;
-    v[KVX] = sx / w;
-    v[KVY] = sy / w;
-    v[KVZ] = sz / w;
+    v[KVX] = sx * iw;
+    v[KVY] = sy * iw;
+    v[KVZ] = sz * iw;
     v[KPR] = pr;
     if (pr <= 0) errcode = 777;
     return errcode;
@@ -1119,8 +1143,9 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
 #pragma unroll
     for (int k = 0; k < NV; k++) uin[k] = gm * u[k];
     d = uin[KRH];
+    const double id = 1. / d;
 #pragma unroll
-    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = uin[k] / uin[KRH];
+    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = uin[k] * id;
     double vx = v[KVX], vy = v[KVY], vz = v[KVZ];
 #pragma unroll
     for (int k = 0; k < NV; k++) vprim[k] = v[k];
@@ -1137,26 +1162,32 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
       s2 = sx * sx_cov + sy * sy_cov + sz * sz_cov;
       pr = v[KPR];
       for (int ip = 1; ip <= 100; ip++) {
-        double qq = en1 + pr;
-        v2 = s2 / (qq * qq);
-        if (v2 >= 1.) return 107;
-        glf = 1. / sqrt(1. - v2);
-        rh = d / glf;
-        en = (en1 + pr) * (1. - v2) - pr - vprim[KPIBU];
-        drhdpr = rh * v2 * glf / (en + pr);
+        w = en1 + pr;
+        iw = rcp_nr(w);
+        v2 = s2 * (iw * iw);
+        if (v2 >= 1. || (w == 0. && s2 > 0.)) return 107;
+        en = w * (1. - v2) - pr - vprim[KPIBU];
+        double drh = 0.;   // dp/drho drho/dp: the ideal gas only
+        if (E.eqstate == 2) {
+          glf = 1. / sqrt(1. - v2);
+          rh = d / glf;
+          drh = rh * v2 * glf / (en + pr);
+        }
         errcode = eos_pressure(E, rh, en, pr_eos, dprdrh, dprden);
         f = pr_eos - pr;
-        df = dprdrh * drhdpr + dprden * v2 - 1.;
-        dpr = -f / df;
+        df = dprdrh * drh + dprden * v2 - 1.;
+        dpr = -quot(f, df);
         if (fabs(dpr) < tol * pr) break;
         pr = pr + dpr;
       }
-      vx = sx / (en1 + pr); if (fabs(vx) < eps) vx = 0.;
-      vy = sy / (en1 + pr); if (fabs(vy) < eps) vy = 0.;
-      vz = sz / (en1 + pr); if (fabs(vz) < eps) vz = 0.;
+      iw = rcp_nr(en1 + pr);
+      vx = sx * iw; if (fabs(vx) < eps) vx = 0.;
+      vy = sy * iw; if (fabs(vy) < eps) vy = 0.;
+      vz = sz * iw; if (fabs(vz) < eps) vz = 0.;
       vprim[KVX] = vx; vprim[KVY] = vy; vprim[KVZ] = vz;
       if (fabs(M.g1 * (vx * vx) + M.g2 * (vy * vy) + M.g3 * (vz * vz) - v2) < eps) break;
     }
+    if (E.eqstate != 2) rh = d * sqrt(1. - v2);
     v[KRH] = rh; v[KVX] = vx; v[KVY] = vy; v[KVZ] = vz; v[KPR] = pr;
     if constexpr (ZZ) derived_pi<true>(v, M);
     return errcode;
@@ -1337,7 +1368,7 @@ __device__ int res_cons2prim(const Eos& E, const Metric& M, const double* u, dou
 __device__ __forceinline__ void ohm_stiff(const Metric& M, const double* vel, const double* Ev, const double* B,
                                           double sig, double sch, double* S) {
   const double v2 = M.g1 * vel[0] * vel[0] + M.g2 * vel[1] * vel[1] + M.g3 * vel[2] * vel[2];
-  const double glf = 1. / sqrt(1. - v2);
+  const double glf = rsqrt_nr(1. - v2);
   double vxB[3], vxE[3];
   cross_contra(M, vel, B, vxB);
   cross_contra(M, vel, Ev, vxE);
@@ -1379,7 +1410,7 @@ __device__ int res_cons2prim_implicit(const Eos& E, const Metric& M, double* u, 
   for (int it = 0; it < 50; it++) {
     const double vel[3] = {v[KVX], v[KVY], v[KVZ]};
     const double v2 = M.g1 * vel[0] * vel[0] + M.g2 * vel[1] * vel[1] + M.g3 * vel[2] * vel[2];
-    const double glf = 1. / sqrt(1. - v2);
+    const double glf = rsqrt_nr(1. - v2);
     const double a = adt * glf * sig, b = adt * glf * sch;
     double vxB[3];
     cross_contra(M, vel, B, vxB);
@@ -1391,7 +1422,7 @@ __device__ int res_cons2prim_implicit(const Eos& E, const Metric& M, double* u, 
     // (1 + a) E - a (v.E) v - b (v x E) = r;  (v x E)^i = C_ij E^j
     const double C[3][3] = {{0., -gp * vel[2], gp * vel[1]},
                             {gp * vel[2], 0., -gp * vel[0]},
-                            {-gp * vel[1] / g3, gp * vel[0] / g3, 0.}};
+                            {-gp * vel[1] * M.ig3, gp * vel[0] * M.ig3, 0.}};
     double m[3][3];
 #pragma unroll
     for (int i = 0; i < 3; i++)
@@ -1400,13 +1431,14 @@ __device__ int res_cons2prim_implicit(const Eos& E, const Metric& M, double* u, 
     const double det = m[0][0] * (m[1][1] * m[2][2] - m[1][2] * m[2][1]) -
                        m[0][1] * (m[1][0] * m[2][2] - m[1][2] * m[2][0]) +
                        m[0][2] * (m[1][0] * m[2][1] - m[1][1] * m[2][0]);
+    const double idet = 1. / det;
     double En[3];
     En[0] = (r[0] * (m[1][1] * m[2][2] - m[1][2] * m[2][1]) - m[0][1] * (r[1] * m[2][2] - m[1][2] * r[2]) +
-             m[0][2] * (r[1] * m[2][1] - m[1][1] * r[2])) / det;
+             m[0][2] * (r[1] * m[2][1] - m[1][1] * r[2])) * idet;
     En[1] = (m[0][0] * (r[1] * m[2][2] - m[1][2] * r[2]) - r[0] * (m[1][0] * m[2][2] - m[1][2] * m[2][0]) +
-             m[0][2] * (m[1][0] * r[2] - r[1] * m[2][0])) / det;
+             m[0][2] * (m[1][0] * r[2] - r[1] * m[2][0])) * idet;
     En[2] = (m[0][0] * (m[1][1] * r[2] - r[1] * m[2][1]) - m[0][1] * (m[1][0] * r[2] - r[1] * m[2][0]) +
-             r[0] * (m[1][0] * m[2][1] - m[1][1] * m[2][0])) / det;
+             r[0] * (m[1][0] * m[2][1] - m[1][1] * m[2][0])) * idet;
     // the change of E against the field scale max(|E|, |B|), not against |E|
     // itself, which can be orders of magnitude smaller than B
     double dE = 0., mE = 0.;

@@ -37,46 +37,26 @@ __device__ __forceinline__ double bulk_zeta(const ViscParams& P, double eta, dou
 
 enum { SXX = 0, SYY = 1, SZZ = 2, SXY = 3, SXZ = 4, SYZ = 5 };
 
-// get_sigma, viscous.f90:283-393 (cell primitives v, derivatives D)
-__device__ __forceinline__ void get_sigma(int coordinates, const Metric& M, const double* v,
-                                          const Deriv& D, double* sigma) {
-  double ux = v[KVX], uy = v[KVY], uz = v[KVZ];
-  double ut = 1. / sqrt(1. - M.g1 * ux * ux - M.g2 * uy * uy - M.g3 * uz * uz);
-  ux = ux * ut; uy = uy * ut; uz = uz * ut;
-  const double dutdt = D.dutdt, duxdx = D.duxdx, duydy = D.duydy, duzdz = D.duzdz;
-  const double duzdt = D.duzdt, duzdx = D.duzdx, duzdy = D.duzdy, duxdt = D.duxdt;
-  const double duxdy = D.duxdy, duxdz = D.duxdz, duydt = D.duydt, duydx = D.duydx, duydz = D.duydz;
-  const double ux2 = ux * ux, uy2 = uy * uy, uz2 = uz * uz;
-  if (coordinates == MINKOWSKI) {
-    sigma[SZZ] = ut * uz * duzdt + uz * ux * duzdx + uz * uy * duzdy + (2. / 3.) * duzdz + (2. / 3.) * duzdz * uz2 - dutdt / 3. - duxdx / 3. - duydy / 3. - uz2 * dutdt / 3.
-                 - uz2 * duxdx / 3. - uz2 * duydy / 3.;
-    sigma[SXZ] = 0.5 * ut * ux * duzdt + 0.5 * duzdx + 0.5 * ux2 * duzdx + 0.5 * ux * uy * duzdy + ux * uz * duzdz / 6. + 0.5 * ut * uz * duxdt + ux * uz * duxdx / 6. + 0.5 * uy * uz *
-                 duxdy + 0.5 * duxdz + 0.5 * duxdz * uz2 - ux * uz * dutdt / 3. - ux * uz * duydy / 3.;
-    sigma[SXY] = 0.5 * ut * ux * duydt + 0.5 * duydx + 0.5 * ux2 * duydx + ux * uy * duydy / 6. + ux * uz * duydz / 2. + 0.5 * ut * uy * duxdt + ux * uy * duxdx / 6. + 0.5 * duxdy +
-                 0.5 * duxdy * uy2 + uy * uz * duxdz / 2. - ux * uy * dutdt / 3. - ux * uy * duzdz / 3.;
-    sigma[SYZ] = 0.5 * ut * uy * duzdt + ux * uy * duzdx / 2. + duzdy / 2. + duzdy * uy2 / 2. + uy * uz * duzdz / 6. + ut * uz * duydt / 2. + ux * uz * duydx / 2. + uy * uz * duydy / 6.
-                 + duydz / 2. + duydz / 2. * uz2 - uy * uz * dutdt / 3. - uy * uz * duxdx / 3.;
-    sigma[SXX] = ut * ux * duxdt + (2. / 3.) * duxdx + (2. / 3.) * duxdx * ux2 + ux * uy * duxdy + ux * uz * duxdz - dutdt / 3. - duydy / 3. - duzdz / 3. - ux2 *
-                 dutdt / 3. - ux2 * duydy / 3. - ux2 * duzdz / 3.;
-    sigma[SYY] = ut * uy * duydt + ux * uy * duydx + (2. / 3.) * duydy + (2. / 3.) * duydy * uy2 + uy * uz * duydz - dutdt / 3. - duxdx / 3. - duzdz / 3. - uy2 *
-                 dutdt / 3. - uy2 * duxdx / 3. - uy2 * duzdz / 3.;
-  } else {
-    const double t = M.t;
-    const double t2 = pow(t, 2.), t3 = t * t * t;   // t**3. as flang lowers it (two multiplications)
-    sigma[SZZ] = ut * uz * duzdt + uz * ux * duzdx + uz * uy * duzdy + (2. * duzdz) / (3. * t2) + (2. / 3.) * duzdz * uz2 - dutdt / (3. * t2) - duxdx / (3. *
-                 t2) - duydy / (3. * t2) - uz2 * dutdt / 3. - uz2 * duxdx / 3. - uz2 * duydy / 3.
-                 + 2. / 3. * ut / t3 + 5. / 3. * (ut / t) * uz2;
-    sigma[SXZ] = 0.5 * ut * ux * duzdt + 0.5 * duzdx + 0.5 * ux2 * duzdx + 0.5 * ux * uy * duzdy + ux * uz * duzdz / 6. + 0.5 * ut * uz * duxdt + ux * uz * duxdx / 6. + 0.5 * uy * uz *
-                 duxdy + duxdz / (2. * t2) + 0.5 * duxdz * uz2 - ux * uz * dutdt / 3. - ux * uz * duydy / 3. + (2. / 3.) * ut * uz * ux / t;
-    sigma[SXY] = 0.5 * ut * ux * duydt + 0.5 * duydx + 0.5 * ux2 * duydx + ux * uy * duydy / 6. + ux * uz * duydz / 2. + 0.5 * ut * uy * duxdt + ux * uy * duxdx / 6. + 0.5 * duxdy +
-                 0.5 * duxdy * uy2 + uy * uz * duxdz / 2. - ux * uy * dutdt / 3. - ux * uy * duzdz / 3. - ut * ux * uy / (3. * t);
-    sigma[SYZ] = 0.5 * ut * uy * duzdt + ux * uy * duzdx / 2. + duzdy / 2. + duzdy * uy2 / 2. + uy * uz * duzdz / 6. + ut * uz * duydt / 2. + ux * uz * duydx / 2. + uy * uz * duydy / 6.
-                 + duydz / (2. * t2) + duydz / 2. * uz2 - uy * uz * dutdt / 3. - uy * uz * duxdx / 3. + (2. / 3.) * ut * uz * uy / t;
-    sigma[SXX] = ut * ux * duxdt + (2. / 3.) * duxdx + (2. / 3.) * duxdx * ux2 + ux * uy * duxdy + ux * uz * duxdz - dutdt / 3. - duydy / 3. - duzdz / 3. - ut / (3. * t) -
-                 ux2 * dutdt / 3. - ux2 * duydy / 3. - ux2 * duzdz / 3. - ux2 * ut / (3. * t);
-    sigma[SYY] = ut * uy * duydt + ux * uy * duydx + (2. / 3.) * duydy + (2. / 3.) * duydy * uy2 + uy * uz * duydz - dutdt / 3. - duxdx / 3. - duzdz / 3. - ut / (3. * t) -
-                 uy2 * dutdt / 3. - uy2 * duxdx / 3. - uy2 * duzdz / 3. - uy2 * ut / (3. * t);
-  }
+// get_sigma, viscous.f90:283-393: the shear tensor of the four-velocity
+// (ut, ux, uy, uz) with derivatives D.  The reference writes every component
+// out; here with the convective derivatives D^i = u^mu d_mu u^i and the
+// expansion theta = d_mu u^mu (+ u^t / t): sigma^ij = (u^i D^j + u^j D^i)/2 +
+// (d_i u^j + d_j u^i)/2 - (g^ij + u^i u^j) theta / 3 and the Bjorken terms, a
+// fifth of the operations.
+__device__ __forceinline__ void get_sigma(int coordinates, const Metric& M, double ut, double ux, double uy,
+                                          double uz, const Deriv& D, double* sigma) {
+  const double Dx = ut * D.duxdt + ux * D.duxdx + uy * D.duxdy + uz * D.duxdz;
+  const double Dy = ut * D.duydt + ux * D.duydx + uy * D.duydy + uz * D.duydz;
+  const double Dz = ut * D.duzdt + ux * D.duzdx + uy * D.duzdy + uz * D.duzdz;
+  const double it = coordinates == MINKOWSKI ? 0. : M.gm;       // 1 / t
+  const double utt = ut * it;
+  const double th3 = (D.dutdt + D.duxdx + D.duydy + D.duzdz + utt) * (1. / 3.);
+  sigma[SXX] = ux * Dx + D.duxdx - (1. + ux * ux) * th3;
+  sigma[SYY] = uy * Dy + D.duydy - (1. + uy * uy) * th3;
+  sigma[SXY] = 0.5 * (ux * Dy + uy * Dx) + 0.5 * (D.duydx + D.duxdy) - ux * uy * th3;
+  sigma[SXZ] = 0.5 * (ux * Dz + uz * Dx) + 0.5 * (D.duzdx + M.ig3 * D.duxdz) - ux * uz * th3 + utt * uz * ux;
+  sigma[SYZ] = 0.5 * (uy * Dz + uz * Dy) + 0.5 * (D.duzdy + M.ig3 * D.duydz) - uy * uz * th3 + utt * uz * uy;
+  sigma[SZZ] = uz * Dz + M.ig3 * D.duzdz - (M.ig3 + uz * uz) * th3 + utt * (it * it + 2. * (uz * uz));
 }
 
 // The EoS values of the viscous source at (rh, pr), with one pressure search
@@ -100,16 +80,16 @@ __device__ __forceinline__ int visc_eos(const Eos& E, double rh, double pr, doub
   const int l = bracket_p(E, pr);
   const double p2 = E.tp[l], p1 = E.tp[l - 1], e2 = E.te[l], e1 = E.te[l - 1];
   const double t2 = E.tt[l], t1 = E.tt[l - 1];
-  en = e1 + (e2 - e1) * (pr - p1) / (p2 - p1);
-  const double f = (pr - p1) / (p2 - p1);
+  const double f = quot(pr - p1, p2 - p1);
   temp = t1 + (t2 - t1) * f;
   const double en2 = e1 + (e2 - e1) * f;
+  en = en2;
   s = (en2 + pr) / temp;
   if (en2 < E.te[0]) { err_sound = 131; return 0; }
   if (en2 > E.te[E.n - 1]) { err_sound = 132; return 0; }
   const int m = (en2 > e1 && en2 < e2) ? l : bracket_e(E, en2);
   const double c2 = E.tc[m], c1 = E.tc[m - 1], g2 = E.te[m], g1 = E.te[m - 1];
-  cs2 = c1 + (c2 - c1) * (en2 - g1) / (g2 - g1);
+  cs2 = c1 + quot((c2 - c1) * (en2 - g1), g2 - g1);
   return 0;
 }
 
@@ -130,7 +110,7 @@ __device__ __forceinline__ int sys_source(const Eos& E, const Metric& M, int coo
   if (err > 0) return err;
   const double t = M.t;
   double v2 = M.g1 * vx * vx + M.g2 * vy * vy + M.g3 * vz * vz;
-  double glf = 1. / sqrt(1. - v2);
+  double glf = rsqrt_nr(1. - v2);
   double ut = glf;
   if constexpr (!VISC) {
     if (coordinates == BJORKEN) {
@@ -149,9 +129,10 @@ __device__ __forceinline__ int sys_source(const Eos& E, const Metric& M, int coo
       }
     }
   } else {
-    const double lambda0 = 1., lambda1 = 1., lambda2 = 0.;
+    // the reference's lambda_0 = lambda_1 = 1; its vorticity terms have the
+    // weight lambda_2 = 0 and are left out
     double sigma[6], eta, zeta, tau_pi;
-    get_sigma(coordinates, M, v, D, sigma);
+    get_sigma(coordinates, M, ut, ut * vx, ut * vy, ut * vz, D, sigma);
     {
       // get_viscous_parameters, viscous.f90:172-199, on the values of visc_eos
       const double HBAR = 0.197326;   // common.f90:47
@@ -163,7 +144,7 @@ __device__ __forceinline__ int sys_source(const Eos& E, const Metric& M, int coo
       err = err_sound;
     }
     if (err > 0) return err;
-    const double tau_pi_big = tau_pi;
+    const double itau = 1. / tau_pi, it = M.gm;   // 1 / t
     PiDer q = derived_pi<ZZ>(v, M);
     const double pitx = q.pitx, pity = q.pity, pitz = q.pitz;
     const double* p = v;
@@ -171,69 +152,56 @@ __device__ __forceinline__ int sys_source(const Eos& E, const Metric& M, int coo
     double sum_der = D.dutdt + D.duxdx + D.duydy + D.duzdz;
     double sum_der_0, sum_der_x, sum_der_y, sum_der_z, sdt;
     if (coordinates == BJORKEN) {
-      sdt = sum_der + ut / t;
+      sdt = sum_der + ut * it;
       sum_der_0 = M.g0 * (glf * D.dutdt + glf * p[KVX] * D.dutdx + glf * p[KVY] * D.dutdy + glf * p[KVZ] * D.dutdz);
       sum_der_x = g1 * (glf * D.duxdt + glf * p[KVX] * D.duxdx + glf * p[KVY] * D.duxdy + glf * p[KVZ] * D.duxdz);
       sum_der_y = g2 * (glf * D.duydt + glf * p[KVX] * D.duydx + glf * p[KVY] * D.duydy + glf * p[KVZ] * D.duydz);
-      sum_der_z = glf * (pow(t, 2.) * D.duzdt + 2. * t * p[KVZ]) + pow(t, 2.) * (glf * p[KVX] * D.duzdx + glf * p[KVY] * D.duzdy + glf * p[KVZ] * D.duzdz);
+      sum_der_z = glf * (g3 * D.duzdt + 2. * t * p[KVZ]) + g3 * (glf * p[KVX] * D.duzdx + glf * p[KVY] * D.duzdy + glf * p[KVZ] * D.duzdz);
       double ww = (en + pr + p[KPIBU]) * (glf * glf);
-      src[KPR] = -t * (ww * vz * vz + (pr + p[KPIBU]) / g3 + p[KPIZZ]);
-      src[KPIBU] = -1. / tau_pi_big * (p[KPIBU] + zeta * sdt) - lambda0 * 4. / 3. * p[KPIBU] * sdt;
+      src[KPR] = -t * (ww * vz * vz + (pr + p[KPIBU]) * M.ig3 + p[KPIZZ]);
+      src[KPIBU] = -itau * (p[KPIBU] + zeta * sdt) - (4. / 3.) * p[KPIBU] * sdt;
     } else {
       sdt = sum_der;
       sum_der_0 = M.g0 * (glf * D.dutdt + p[KVX] * D.dutdx + p[KVY] * D.dutdy + p[KVZ] * D.dutdz);
       sum_der_x = g1 * (glf * D.duxdt + p[KVX] * D.duxdx + p[KVY] * D.duxdy + p[KVZ] * D.duxdz);
       sum_der_y = g2 * (glf * D.duydt + p[KVX] * D.duydx + p[KVY] * D.duydy + p[KVZ] * D.duydz);
       sum_der_z = g3 * (glf * D.duzdt + p[KVX] * D.duzdx + p[KVY] * D.duzdy + p[KVZ] * D.duzdz);
-      src[KPIBU] = -1. / tau_pi_big * (p[KPIBU] + zeta * sum_der) + lambda0 * (-1. / 3. * p[KPIBU] * sum_der);
+      src[KPIBU] = -itau * (p[KPIBU] + zeta * sum_der) + (-1. / 3. * p[KPIBU] * sum_der);
     }
-    double w0x = -0.5 * (D.dutdx + D.duxdt) + 0.5 * glf * (sum_der_x - p[KVX] * g1 * sum_der_0);
-    double w0y = -0.5 * (D.dutdy + D.duydt) + 0.5 * glf * (sum_der_y - p[KVY] * g2 * sum_der_0);
-    double w0z = -0.5 * (D.dutdz + D.duzdt) + 0.5 * glf * (sum_der_z - p[KVZ] * g3 * sum_der_0);
-    double wxy = 0.5 * (g2 * D.duydx - D.duxdy) + 0.5 * glf * (g1 * p[KVX] * sum_der_y - g2 * p[KVY] * sum_der_x);
-    double wxz = 0.5 * (g3 * D.duzdx - D.duxdz) + 0.5 * glf * (g1 * p[KVX] * sum_der_z - g3 * p[KVZ] * sum_der_x);
-    double wyz = 0.5 * (g3 * D.duzdy - D.duydz) + 0.5 * glf * (g2 * p[KVY] * sum_der_z - g3 * p[KVZ] * sum_der_y);
-    double wx0 = w0x, wy0 = w0y, wz0 = w0z, wyx = -wxy, wzx = -wxz, wzy = -wyz;
-    double IVxx = 2. * (pitx * wx0 + p[KPIXY] * wxy + p[KPIXZ] * wxz);
-    double IVyy = 2. * (pity * wy0 + p[KPIXY] * wyx + p[KPIYZ] * wyz);
-    double IVzz = 2. * (pitz * wz0 + p[KPIXZ] * wzx + p[KPIYZ] * wzy);
-    double IVxy = p[KPIXX] * wyx + p[KPIYY] * wxy + p[KPIXZ] * wyz + p[KPIYZ] * wxz + pitx * wy0 + pity * wx0;
-    double IVxz = p[KPIXX] * wzx + p[KPIZZ] * wxz + p[KPIXY] * wzy + p[KPIYZ] * wxy + pitx * wz0 + pitz * wx0;
-    double IVyz = p[KPIYY] * wzy + p[KPIZZ] * wyz + p[KPIXY] * wzx + p[KPIXZ] * wyx + pity * wz0 + pitz * wy0;
     if (coordinates == BJORKEN) {
       const double sum_der_t = sdt;
-      src[KPIZZ] = -1. / tau_pi * (p[KPIZZ] + 2. * eta * sigma[SZZ]) - 2. * glf * p[KPIZZ] / t -
-                   2. * (glf * vz) * pitz / t - lambda0 * 4. / 3. * p[KPIZZ] * sum_der_t + lambda1 * glf * (2. * p[KVZ] * (pitz * sum_der_0 +
-                   p[KPIXZ] * sum_der_x + p[KPIYZ] * sum_der_y + p[KPIZZ] * sum_der_z)) - lambda2 * IVzz;
-      src[KPIXZ] = -1. / tau_pi * (p[KPIXZ] + 2. * eta * sigma[SXZ]) + lambda0 * (-4. / 3. * p[KPIXZ] * sum_der_t) - glf / t * p[KPIXZ] - glf * vz * pitx / t +
-                   lambda1 * glf * ((pitx * p[KVZ] + pitz * p[KVX]) * sum_der_0 + (p[KPIXX] * p[KVZ] + p[KPIXZ] * p[KVX]) * sum_der_x + (p[KPIXY] * p[KVZ] +
-                   p[KPIYZ] * p[KVX]) * sum_der_y + (p[KPIXZ] * p[KVZ] + p[KPIZZ] * p[KVX]) * sum_der_z) - lambda2 * IVxz;
-      src[KPIYZ] = -1. / tau_pi * (p[KPIYZ] + 2. * eta * sigma[SYZ]) + lambda0 * (-4. / 3. * p[KPIYZ] * sum_der_t) - glf / t * p[KPIYZ] - glf * vz * pity / t +
-                   lambda1 * glf * ((pity * p[KVZ] + pitz * p[KVY]) * sum_der_0 + (p[KPIXY] * p[KVZ] + p[KPIXZ] * p[KVY]) * sum_der_x + (p[KPIYY] * p[KVZ] +
-                   p[KPIYZ] * p[KVY]) * sum_der_y + (p[KPIYZ] * p[KVZ] + p[KPIZZ] * p[KVY]) * sum_der_z) - lambda2 * IVyz;
-      src[KPIXY] = -1. / tau_pi * (p[KPIXY] + 2. * eta * sigma[SXY]) + lambda0 * (-4. / 3. * p[KPIXY] * sum_der_t) + lambda1 * glf * ((pitx *
+      src[KPIZZ] = -itau * (p[KPIZZ] + 2. * eta * sigma[SZZ]) - 2. * glf * p[KPIZZ] * it -
+                   2. * (glf * vz) * pitz * it - (4. / 3.) * p[KPIZZ] * sum_der_t + glf * (2. * p[KVZ] * (pitz * sum_der_0 +
+                   p[KPIXZ] * sum_der_x + p[KPIYZ] * sum_der_y + p[KPIZZ] * sum_der_z));
+      src[KPIXZ] = -itau * (p[KPIXZ] + 2. * eta * sigma[SXZ]) + (-4. / 3. * p[KPIXZ] * sum_der_t) - glf * it * p[KPIXZ] - glf * vz * pitx * it +
+                   glf * ((pitx * p[KVZ] + pitz * p[KVX]) * sum_der_0 + (p[KPIXX] * p[KVZ] + p[KPIXZ] * p[KVX]) * sum_der_x + (p[KPIXY] * p[KVZ] +
+                   p[KPIYZ] * p[KVX]) * sum_der_y + (p[KPIXZ] * p[KVZ] + p[KPIZZ] * p[KVX]) * sum_der_z);
+      src[KPIYZ] = -itau * (p[KPIYZ] + 2. * eta * sigma[SYZ]) + (-4. / 3. * p[KPIYZ] * sum_der_t) - glf * it * p[KPIYZ] - glf * vz * pity * it +
+                   glf * ((pity * p[KVZ] + pitz * p[KVY]) * sum_der_0 + (p[KPIXY] * p[KVZ] + p[KPIXZ] * p[KVY]) * sum_der_x + (p[KPIYY] * p[KVZ] +
+                   p[KPIYZ] * p[KVY]) * sum_der_y + (p[KPIYZ] * p[KVZ] + p[KPIZZ] * p[KVY]) * sum_der_z);
+      src[KPIXY] = -itau * (p[KPIXY] + 2. * eta * sigma[SXY]) + (-4. / 3. * p[KPIXY] * sum_der_t) + glf * ((pitx *
                    p[KVY] + pity * p[KVX]) * sum_der_0 + (p[KPIXX] * p[KVY] + p[KPIXY] * p[KVX]) * sum_der_x + (p[KPIXY] * p[KVY] + p[KPIYY] * p[KVX]) *
-                   sum_der_y + (p[KPIXZ] * p[KVY] + p[KPIYZ] * p[KVX]) * sum_der_z) - lambda2 * IVxy;
-      src[KPIXX] = -1. / tau_pi * (p[KPIXX] + 2. * eta * sigma[SXX]) + lambda0 * (-4. / 3. * p[KPIXX] * sum_der_t) + lambda1 * glf * (2. * p[KVX] * (pitx *
-                   sum_der_0 + p[KPIXX] * sum_der_x + p[KPIXY] * sum_der_y + p[KPIXZ] * sum_der_z)) - lambda2 * IVxx;
-      src[KPIYY] = -1. / tau_pi * (p[KPIYY] + 2. * eta * sigma[SYY]) + lambda0 * (-4. / 3. * p[KPIYY] * sum_der_t) + lambda1 * glf * (2. * p[KVY] * (pity *
-                   sum_der_0 + p[KPIXY] * sum_der_x + p[KPIYY] * sum_der_y + p[KPIYZ] * sum_der_z)) - lambda2 * IVyy;
+                   sum_der_y + (p[KPIXZ] * p[KVY] + p[KPIYZ] * p[KVX]) * sum_der_z);
+      src[KPIXX] = -itau * (p[KPIXX] + 2. * eta * sigma[SXX]) + (-4. / 3. * p[KPIXX] * sum_der_t) + glf * (2. * p[KVX] * (pitx *
+                   sum_der_0 + p[KPIXX] * sum_der_x + p[KPIXY] * sum_der_y + p[KPIXZ] * sum_der_z));
+      src[KPIYY] = -itau * (p[KPIYY] + 2. * eta * sigma[SYY]) + (-4. / 3. * p[KPIYY] * sum_der_t) + glf * (2. * p[KVY] * (pity *
+                   sum_der_0 + p[KPIXY] * sum_der_x + p[KPIYY] * sum_der_y + p[KPIYZ] * sum_der_z));
     } else {
-      src[KPIZZ] = -1. / tau_pi * (p[KPIZZ] + 2. * eta * sigma[SZZ]) + lambda0 * (-4. / 3. * p[KPIZZ] * sum_der) + lambda1 * (2. * p[KVZ] * (pitz * sum_der_0
-                   + p[KPIXZ] * sum_der_x + p[KPIYZ] * sum_der_y + p[KPIZZ] * sum_der_z)) - lambda2 * IVzz;
-      src[KPIXZ] = -1. / tau_pi * (p[KPIXZ] + 2. * eta * sigma[SXZ]) + lambda0 * (-4. / 3. * p[KPIXZ] * sum_der) + lambda1 * ((pitx * p[KVZ] + pitz * p[KVX]) *
+      src[KPIZZ] = -itau * (p[KPIZZ] + 2. * eta * sigma[SZZ]) + (-4. / 3. * p[KPIZZ] * sum_der) + (2. * p[KVZ] * (pitz * sum_der_0
+                   + p[KPIXZ] * sum_der_x + p[KPIYZ] * sum_der_y + p[KPIZZ] * sum_der_z));
+      src[KPIXZ] = -itau * (p[KPIXZ] + 2. * eta * sigma[SXZ]) + (-4. / 3. * p[KPIXZ] * sum_der) + ((pitx * p[KVZ] + pitz * p[KVX]) *
                    sum_der_0 + (p[KPIXX] * p[KVZ] + p[KPIXZ] * p[KVX]) * sum_der_x + (p[KPIXY] * p[KVZ] + p[KPIYZ] * p[KVX]) * sum_der_y + (p[KPIXZ] * p[KVZ]
-                   + p[KPIZZ] * p[KVX]) * sum_der_z) - lambda2 * IVxz;
-      src[KPIXY] = -1. / tau_pi * (p[KPIXY] + 2. * eta * sigma[SXY]) + lambda0 * (-4. / 3. * p[KPIXY] * sum_der) + lambda1 * ((pitx * p[KVY] + pity * p[KVX]) *
+                   + p[KPIZZ] * p[KVX]) * sum_der_z);
+      src[KPIXY] = -itau * (p[KPIXY] + 2. * eta * sigma[SXY]) + (-4. / 3. * p[KPIXY] * sum_der) + ((pitx * p[KVY] + pity * p[KVX]) *
                    sum_der_0 + (p[KPIXX] * p[KVY] + p[KPIXY] * p[KVX]) * sum_der_x + (p[KPIXY] * p[KVY] + p[KPIYY] * p[KVX]) * sum_der_y + (p[KPIXZ] * p[KVY]
-                   + p[KPIYZ] * p[KVX]) * sum_der_z) - lambda2 * IVxy;
-      src[KPIYZ] = -1. / tau_pi * (p[KPIYZ] + 2. * eta * sigma[SYZ]) + lambda0 * (-4. / 3. * p[KPIYZ] * sum_der) + lambda1 * ((pity * p[KVZ] + pitz * p[KVY]) *
+                   + p[KPIYZ] * p[KVX]) * sum_der_z);
+      src[KPIYZ] = -itau * (p[KPIYZ] + 2. * eta * sigma[SYZ]) + (-4. / 3. * p[KPIYZ] * sum_der) + ((pity * p[KVZ] + pitz * p[KVY]) *
                    sum_der_0 + (p[KPIXY] * p[KVZ] + p[KPIXZ] * p[KVY]) * sum_der_x + (p[KPIYY] * p[KVZ] + p[KPIYZ] * p[KVY]) * sum_der_y + (p[KPIYZ] * p[KVZ]
-                   + p[KPIZZ] * p[KVY]) * sum_der_z) - lambda2 * IVyz;
-      src[KPIXX] = -1. / tau_pi * (p[KPIXX] + 2. * eta * sigma[SXX]) + lambda0 * (-4. / 3. * p[KPIXX] * sum_der) + lambda1 * (2. * p[KVX] * (pitx * sum_der_0 +
-                   p[KPIXX] * sum_der_x + p[KPIXY] * sum_der_y + p[KPIXZ] * sum_der_z)) - lambda2 * IVxx;
-      src[KPIYY] = -1. / tau_pi * (p[KPIYY] + 2. * eta * sigma[SYY]) + lambda0 * (-4. / 3. * p[KPIYY] * sum_der) + lambda1 * (2. * p[KVY] * (pity * sum_der_0 +
-                   p[KPIXY] * sum_der_x + p[KPIYY] * sum_der_y + p[KPIYZ] * sum_der_z)) - lambda2 * IVyy;
+                   + p[KPIZZ] * p[KVY]) * sum_der_z);
+      src[KPIXX] = -itau * (p[KPIXX] + 2. * eta * sigma[SXX]) + (-4. / 3. * p[KPIXX] * sum_der) + (2. * p[KVX] * (pitx * sum_der_0 +
+                   p[KPIXX] * sum_der_x + p[KPIXY] * sum_der_y + p[KPIXZ] * sum_der_z));
+      src[KPIYY] = -itau * (p[KPIYY] + 2. * eta * sigma[SYY]) + (-4. / 3. * p[KPIYY] * sum_der) + (2. * p[KVY] * (pity * sum_der_0 +
+                   p[KPIXY] * sum_der_x + p[KPIYY] * sum_der_y + p[KPIYZ] * sum_der_z));
     }
 #pragma unroll
     for (int k = KPIBU; k < NV; k++) src[k] = src[k] * v[KRH];
