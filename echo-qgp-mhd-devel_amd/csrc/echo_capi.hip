@@ -32,24 +32,46 @@ static void rk_coeffs(int nrk, int irk, double& c1, double& c2) {
 // of echo_set_tile
 static int flux_tx(int ty) { return ty == 1 ? 16 : ty == 2 ? 32 : 8; }
 
-// flux launch of one sweep with the grid's tile shape
-template <int DIR, int REC, int SYS, bool ZZ>
-static void launch_flux_rec(echo_grid* g, double* partial) {
-  k_flux<DIR, REC, SYS, ZZ><<<g->nb[DIR - 1], FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, g->F[DIR - 1], g->L[DIR - 1],
-                                                                          partial, flux_tx(g->tile[DIR - 1]));
+// blocks of a sweep, 0 for a dimension with one cell
+static unsigned sweep_blocks(const echo_grid* g, int d) { return g->active[d] ? (unsigned)g->nb[d] : 0u; }
+
+// flux launch of the sweeps in `dirs` (bit d for direction d) with the grid's
+// tile shapes
+template <int SYS, bool ZZ>
+static void launch_flux(echo_grid* g, unsigned dirs) {
+  FluxBufs b;
+  unsigned n = 0, off = 0;
+  for (int d = 0; d < 3; d++) {
+    b.partial[d] = g->partial + off;
+    off += sweep_blocks(g, d);
+    b.F[d] = g->F[d];
+    b.L[d] = g->L[d];
+    b.tx[d] = flux_tx(g->tile[d]);
+    b.nb[d] = dirs >> d & 1 ? sweep_blocks(g, d) : 0;
+    n += b.nb[d];
+  }
+  if (!n) return;
+  switch (g->cfg.recal) {
+    case REC_TVD2: k_flux<REC_TVD2, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    case REC_CENO3: k_flux<REC_CENO3, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    case REC_WENO3: k_flux<REC_WENO3, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    case REC_PPM4: k_flux<REC_PPM4, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    case REC_MPE3: k_flux<REC_MPE3, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    case REC_MPE5: k_flux<REC_MPE5, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+    default: k_flux<REC_WENO5, SYS, ZZ><<<n, FLUX_BLOCK, 0, g->stream>>>(g->ga, g->V, b); break;
+  }
 }
 
-template <int DIR, int SYS, bool ZZ>
-static void launch_flux_dir(echo_grid* g, double* partial) {
-  switch (g->cfg.recal) {
-    case REC_TVD2: launch_flux_rec<DIR, REC_TVD2, SYS, ZZ>(g, partial); break;
-    case REC_CENO3: launch_flux_rec<DIR, REC_CENO3, SYS, ZZ>(g, partial); break;
-    case REC_WENO3: launch_flux_rec<DIR, REC_WENO3, SYS, ZZ>(g, partial); break;
-    case REC_PPM4: launch_flux_rec<DIR, REC_PPM4, SYS, ZZ>(g, partial); break;
-    case REC_MPE3: launch_flux_rec<DIR, REC_MPE3, SYS, ZZ>(g, partial); break;
-    case REC_MPE5: launch_flux_rec<DIR, REC_MPE5, SYS, ZZ>(g, partial); break;
-    default: launch_flux_rec<DIR, REC_WENO5, SYS, ZZ>(g, partial); break;
+// The sweeps of a stage: one launch; with kernel timing one per sweep, between
+// the events ev[0..3].
+template <int SYS, bool ZZ>
+static void launch_sweeps(echo_grid* g) {
+  if (!g->timing) return launch_flux<SYS, ZZ>(g, 7u);
+  for (int d = 0; d < 3; d++) {
+    hipEventRecord(g->ev[d], g->stream);
+    launch_flux<SYS, ZZ>(g, 1u << d);
   }
+  hipEventRecord(g->ev[3], g->stream);
 }
 
 // launch blocks of a sweep for tile shape ty (padded for xcd_block)
@@ -75,16 +97,10 @@ static void enqueue_stage_t(echo_grid* g, int irk) {
   const int nrk = g->cfg.nrk;
   double c1, c2;
   rk_coeffs(nrk, irk, c1, c2);
-  double* part[3] = {g->partial, g->partial + g->nb[0], g->partial + g->nb[0] + g->nb[1]};
-  if (g->timing) hipEventRecord(g->ev[0], g->stream);
-  if (g->active[0]) launch_flux_dir<1, SYS, ZZ>(g, part[0]);
-  if (g->timing) hipEventRecord(g->ev[1], g->stream);
-  if (g->active[1]) launch_flux_dir<2, SYS, ZZ>(g, part[1]);
-  if (g->timing) hipEventRecord(g->ev[2], g->stream);
-  if (g->active[2]) launch_flux_dir<3, SYS, ZZ>(g, part[2]);
-  if (g->timing) hipEventRecord(g->ev[3], g->stream);
+  launch_sweeps<SYS, ZZ>(g);
   if (irk == 1) {
-    k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, g->nb[0], g->nb[1], g->nb[2]);
+    k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
+                                       sweep_blocks(g, 2));
   }
   if (g->timing) hipEventRecord(g->ev[4], g->stream);
   // stage 1 reads u^n from U[0] and writes U[1]; later stages update U[1]
@@ -119,21 +135,15 @@ static void enqueue_stage_t(echo_grid* g, int irk) {
 template <int SYS, bool ZZ>
 static void enqueue_imex_stage_t(echo_grid* g, int irk) {
   if constexpr (!SysT<SYS>::RES) {
-    double* part[3] = {g->partial, g->partial + g->nb[0], g->partial + g->nb[0] + g->nb[1]};
     double* Ust = g->U[1];
     auto fixup = [&](double* U, int last, int phase) {
       k_fixup<SYS, ZZ><<<1, FIX_BLOCK, 0, g->stream>>>(g->ga, g->V, U, g->fix, g->VS[0], g->VS[1], last,
                                                         ImexView{g->U[0], g->imex.P4, phase}, last);
     };
-    if (g->timing) hipEventRecord(g->ev[0], g->stream);
-    if (g->active[0]) launch_flux_dir<1, SYS, ZZ>(g, part[0]);
-    if (g->timing) hipEventRecord(g->ev[1], g->stream);
-    if (g->active[1]) launch_flux_dir<2, SYS, ZZ>(g, part[1]);
-    if (g->timing) hipEventRecord(g->ev[2], g->stream);
-    if (g->active[2]) launch_flux_dir<3, SYS, ZZ>(g, part[2]);
-    if (g->timing) hipEventRecord(g->ev[3], g->stream);
+    launch_sweeps<SYS, ZZ>(g);
     // dt from the speeds of the step's first sweeps, as in the RK steps
-    if (irk == 1) k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, g->nb[0], g->nb[1], g->nb[2]);
+    if (irk == 1) k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
+                                       sweep_blocks(g, 2));
     if (g->timing) hipEventRecord(g->ev[4], g->stream);
     if (irk == 1) {
       // K2 = u0 (evolve.f90:232-233): its inversion; the repair also sets
@@ -157,7 +167,6 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
     else fixup(Ust, 0, irk + 1);
   } else {
     const unsigned nbu = nblocks_xcd(g->N, UPDATE_BLOCK);
-    double* part[3] = {g->partial, g->partial + g->nb[0], g->partial + g->nb[0] + g->nb[1]};
     double* Ust = g->U[1];
     // the repair after the implicit solve of K_phase (phase 0: the step's
     // result), reading U* through ImexView
@@ -168,7 +177,8 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
     if (g->timing) hipEventRecord(g->ev[0], g->stream);
     if (irk == 1) {
       if (g->timing) for (int i = 1; i < 4; i++) hipEventRecord(g->ev[i], g->stream);
-      k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, g->nb[0], g->nb[1], g->nb[2]);
+      k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
+                                       sweep_blocks(g, 2));
       if (g->timing) hipEventRecord(g->ev[4], g->stream);
       k_imex_k1<SYS, ZZ><<<nbu, UPDATE_BLOCK, 0, g->stream>>>(g->ga, g->V, g->U[0], Ust, g->fix);
       fixup(Ust, 0, 1);
@@ -177,15 +187,8 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
       fixup(Ust, 0, 2);
       return;
     }
-    if (g->active[0]) launch_flux_dir<1, SYS, ZZ>(g, part[0]);
-    if (g->timing) hipEventRecord(g->ev[1], g->stream);
-    if (g->active[1]) launch_flux_dir<2, SYS, ZZ>(g, part[1]);
-    if (g->timing) hipEventRecord(g->ev[2], g->stream);
-    if (g->active[2]) launch_flux_dir<3, SYS, ZZ>(g, part[2]);
-    if (g->timing) {
-      hipEventRecord(g->ev[3], g->stream);
-      hipEventRecord(g->ev[4], g->stream);
-    }
+    launch_sweeps<SYS, ZZ>(g);
+    if (g->timing) hipEventRecord(g->ev[4], g->stream);
 #define ECHO_IMEX_UPDATE(ST)                                                                        \
   k_update_imex<SYS, ZZ, ST><<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(                    \
       g->ga, g->V, g->U[0], Ust, g->F[0], g->F[1], g->F[2], g->L[0], g->L[1], g->L[2], g->VS[0], \
@@ -211,14 +214,7 @@ static void enqueue_stage(echo_grid* g, int irk) {
 
 // one flux sweep (direction d = 0, 1, 2) with the current tile shape
 static void enqueue_flux(echo_grid* g, int d) {
-  double* part[3] = {g->partial, g->partial + g->nb[0], g->partial + g->nb[0] + g->nb[1]};
-  dispatch_sys(g->cfg, [&](auto sys, auto zz) {
-    constexpr int S = decltype(sys)::value;
-    constexpr bool Z = decltype(zz)::value;
-    if (d == 0) launch_flux_dir<1, S, Z>(g, part[0]);
-    else if (d == 1) launch_flux_dir<2, S, Z>(g, part[1]);
-    else launch_flux_dir<3, S, Z>(g, part[2]);
-  });
+  dispatch_sys(g->cfg, [&](auto sys, auto zz) { launch_flux<decltype(sys)::value, decltype(zz)::value>(g, 1u << d); });
 }
 
 static int set_tile(echo_grid* g, int d, int ty) {

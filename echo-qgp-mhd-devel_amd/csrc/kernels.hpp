@@ -220,17 +220,35 @@ __device__ __forceinline__ void block_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// buffers of the three sweeps and their share of a launch: block counts (0 for
+// a sweep that does not run), and the columns tx of the y and z tiles
+struct FluxBufs {
+  double* F[3];
+  double* L[3];
+  double* partial[3];
+  unsigned nb[3];
+  int tx[3];
+};
+
+template <int SYS>
+struct FluxLds {
+  static constexpr int NI = SysT<SYS>::NV + (SysT<SYS>::VISC ? 4 : 0);
+  static constexpr int GS = flux_group<SYS>(), NG = (NI + GS - 1) / GS, NBUF = NG > 1 ? 2 : 1;
+  double sw[SysT<SYS>::NV][FLUX_BLOCK];
+  double st[NBUF][GS][FLUX_STAGE];
+  double red[FLUX_BLOCK / 64];
+};
+
 template <int DIR, int REC, int SYS, bool ZZ>
-__global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs a, const double* __restrict__ V,
-                                                     double* __restrict__ F, double* __restrict__ L,
-                                                     double* __restrict__ partial, int tx) {
+__device__ __forceinline__ void flux_block(const GridArgs& a, const double* __restrict__ V, double* __restrict__ F,
+                                           double* __restrict__ L, double* __restrict__ partial, unsigned block,
+                                           unsigned nblocks, int tx, FluxLds<SYS>& lds) {
   constexpr bool VISC = SysT<SYS>::VISC;
   constexpr int NV = SysT<SYS>::NV;
-  if (a.S->temp_check) return;   // the run has stopped (check_temp)
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const int m = DIR == 1 ? nx : (DIR == 2 ? ny : nz);
   const unsigned t = threadIdx.x;
-  const unsigned tile = (unsigned)xcd_block(blockIdx.x, gridDim.x);
+  const unsigned tile = (unsigned)xcd_block(block, nblocks);
   // the thread's cell: index ci along the sweep (-1 .. m), and whether it owns
   // its upper interface, number ci + 1 of the line, f in the face array.
   // Threads without a cell work on values of other cells up to the exchange.
@@ -285,10 +303,10 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
   // gamma v^i), reconstructed for deriv (evolve.f90:324-331, 371-374); it is
   // formed once per staged cell.
   constexpr int NU = VISC ? 4 : 0, NI = NV + NU;
-  constexpr int GS = flux_group<SYS>(), NG = (NI + GS - 1) / GS, NBUF = NG > 1 ? 2 : 1;
+  constexpr int GS = FluxLds<SYS>::GS, NG = FluxLds<SYS>::NG, NBUF = FluxLds<SYS>::NBUF;
   static_assert(!VISC || (GS == 4 && NG >= 4), "the Lorentz velocity's lower states wait in the last group's slots");
-  __shared__ double sw[NV][FLUX_BLOCK];
-  __shared__ double st[NBUF][GS][FLUX_STAGE];
+  auto& sw = lds.sw;
+  auto& st = lds.st;
   const unsigned tr = t + up < FLUX_BLOCK ? t + up : t;
   // staged positions: p = t and, for the first 4 * up threads, p = FLUX_BLOCK + t
   const bool second = t < 4u * up;
@@ -525,26 +543,42 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
       if constexpr (SysT<SYS>::RES) __builtin_nontemporal_store(dEface, &F[(long long)NV * nf + f]);
     }
   }
-  // block max of the interface speeds -> partial[blockIdx.x]
-  __shared__ double red[FLUX_BLOCK / 64];
+  // block max of the interface speeds
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) amax = dmax(amax, __shfl_xor(amax, o, 64));
-  if ((t & 63) == 0) red[t >> 6] = amax;
+  if ((t & 63) == 0) lds.red[t >> 6] = amax;
   __syncthreads();
   if (t == 0) {
-    double r = red[0];
+    double r = lds.red[0];
 #pragma unroll
-    for (int w = 1; w < FLUX_BLOCK / 64; w++) r = dmax(r, red[w]);
-    partial[blockIdx.x] = r;
+    for (int w = 1; w < FLUX_BLOCK / 64; w++) r = dmax(r, lds.red[w]);
+    partial[block] = r;
   }
+}
+
+// The sweeps of a stage in one launch (they are independent): blocks [0, nb0)
+// are the x sweep's, the next nb1 the y sweep's, the rest the z sweep's.  On
+// small grids a sweep alone does not fill the chip and takes little more than
+// a launch; large ones lose two tails per stage.
+template <int REC, int SYS, bool ZZ>
+__global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs a, const double* __restrict__ V,
+                                                                      FluxBufs b) {
+  __shared__ FluxLds<SYS> lds;
+  if (a.S->temp_check) return;   // the run has stopped (check_temp)
+  unsigned i = blockIdx.x;
+  if (i < b.nb[0]) return flux_block<1, REC, SYS, ZZ>(a, V, b.F[0], b.L[0], b.partial[0], i, b.nb[0], b.tx[0], lds);
+  i -= b.nb[0];
+  if (i < b.nb[1])
+    return flux_block<2, REC, SYS, ZZ>(a, V, b.F[1], b.L[1], b.partial[1], i, b.nb[1], b.tx[1], lds);
+  i -= b.nb[1];
+  flux_block<3, REC, SYS, ZZ>(a, V, b.F[2], b.L[2], b.partial[2], i, b.nb[2], b.tx[2], lds);
 }
 
 // ---------------------------------------------------------------------------
 // k_cfl: reduces the per-block speed maxima of the three sweeps and applies
 // evolve_dt (evolve.f90:723-764) and the clamps of evolve.f90:179-188.
 // One block.  partial holds nb0 + nb1 + nb2 values (the block counts of the
-// three sweeps, in this order); only the sweeps of active dimensions
-// (n > 1) wrote theirs.
+// three sweeps, in this order, 0 for those of dimensions with one cell).
 // ---------------------------------------------------------------------------
 static __global__ __launch_bounds__(1024) void k_cfl(GridArgs a, const double* __restrict__ partial,
                                               int nb0, int nb1, int nb2) {
