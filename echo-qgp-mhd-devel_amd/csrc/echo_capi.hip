@@ -38,8 +38,9 @@ static unsigned sweep_blocks(const echo_grid* g, int d) { return g->active[d] ? 
 // flux launch of the sweeps in `dirs` (bit d for direction d) with the grid's
 // tile shapes
 template <int SYS, bool ZZ>
-static void launch_flux(echo_grid* g, unsigned dirs) {
+static void launch_flux(echo_grid* g, unsigned dirs, int irk) {
   FluxBufs b;
+  b.irk = irk;
   unsigned n = 0, off = 0;
   for (int d = 0; d < 3; d++) {
     b.partial[d] = g->partial + off;
@@ -65,11 +66,11 @@ static void launch_flux(echo_grid* g, unsigned dirs) {
 // The sweeps of a stage: one launch; with kernel timing one per sweep, between
 // the events ev[0..3].
 template <int SYS, bool ZZ>
-static void launch_sweeps(echo_grid* g) {
-  if (!g->timing) return launch_flux<SYS, ZZ>(g, 7u);
+static void launch_sweeps(echo_grid* g, int irk) {
+  if (!g->timing) return launch_flux<SYS, ZZ>(g, 7u, irk);
   for (int d = 0; d < 3; d++) {
     hipEventRecord(g->ev[d], g->stream);
-    launch_flux<SYS, ZZ>(g, 1u << d);
+    launch_flux<SYS, ZZ>(g, 1u << d, irk);
   }
   hipEventRecord(g->ev[3], g->stream);
 }
@@ -92,16 +93,30 @@ static unsigned update_blocks(const echo_grid* g) {
   return (unsigned)((t + NXCD - 1) / NXCD * NXCD);
 }
 
+// per-block speed maxima of the grid's sweeps
+static SpeedMax speed_max(const echo_grid* g) {
+  return SpeedMax{g->partial, {sweep_blocks(g, 0), sweep_blocks(g, 1), sweep_blocks(g, 2)}};
+}
+
+// con2prim repair of the cells that stage irk could not invert (rare; returns
+// at once when there are none); it writes the next step's vnewstep too,
+// before k_end_step flips the parity
 template <int SYS, bool ZZ>
-static void enqueue_stage_t(echo_grid* g, int irk) {
+static void enqueue_fixup_t(echo_grid* g, int irk) {
+  const bool last = irk == g->cfg.nrk;
+  k_fixup<SYS, ZZ><<<1, FIX_BLOCK, 0, g->stream>>>(g->ga, g->V, last ? g->U[0] : g->U[1], g->fix, g->VS[0], g->VS[1],
+                                                    last ? 1 : 0, ImexView{nullptr, nullptr, 0}, 1);
+}
+
+template <int SYS, bool ZZ>
+static void enqueue_stage_t(echo_grid* g, int irk, bool fixup) {
   const int nrk = g->cfg.nrk;
   double c1, c2;
   rk_coeffs(nrk, irk, c1, c2);
-  launch_sweeps<SYS, ZZ>(g);
-  if (irk == 1) {
-    k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
-                                       sweep_blocks(g, 2));
-  }
+  launch_sweeps<SYS, ZZ>(g, irk);
+  const SpeedMax speeds = speed_max(g);
+  const bool cfl = irk == 1 && speeds.nb[0] + speeds.nb[1] + speeds.nb[2] <= CFL_IN_UPDATE;
+  if (irk == 1 && !cfl) k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, speeds);
   if (g->timing) hipEventRecord(g->ev[4], g->stream);
   // stage 1 reads u^n from U[0] and writes U[1]; later stages update U[1]
   // in place; the last stage writes u^{n+1} back into U[0] (each cell reads
@@ -110,17 +125,15 @@ static void enqueue_stage_t(echo_grid* g, int irk) {
   double* Ucur = (irk == 1) ? g->U[0] : g->U[1];
   double* Uout = last ? g->U[0] : g->U[1];
   dispatch_algo<SYS>(g->cfg, [&](auto algo) {
-    k_update<SYS, ZZ, decltype(algo)::value><<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(
+    constexpr int A = decltype(algo)::value;
+    auto* kernel = cfl ? k_update<SYS, ZZ, A, true> : k_update<SYS, ZZ, A, false>;
+    kernel<<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(
         g->ga, g->V, g->U[0], Ucur, Uout, g->F[0], g->F[1], g->F[2], g->L[0], g->L[1], g->L[2],
-        g->VS[0], g->VS[1], g->fix, c1, c2, irk == 1 ? 1 : 0, last ? 1 : 0);
+        g->VS[0], g->VS[1], g->fix, StageArgs{c1, c2, speeds, irk, last ? 1 : 0});
   });
   if (g->net) enqueue_net_c2p(g, Uout);   // ideal MHD with the learned inversion
   if (g->timing) hipEventRecord(g->ev[5], g->stream);
-  // con2prim repair of the cells k_update could not invert (rare; returns at
-  // once when there are none); it writes the next step's vnewstep too,
-  // before k_end_step flips the parity
-  k_fixup<SYS, ZZ><<<1, FIX_BLOCK, 0, g->stream>>>(g->ga, g->V, Uout, g->fix, g->VS[0],
-                                                    g->VS[1], last ? 1 : 0, ImexView{nullptr, nullptr, 0}, 1);
+  if (fixup) enqueue_fixup_t<SYS, ZZ>(g, irk);
 }
 
 // one stage of IMEX-SSP3(4,3,3) (kernels.hpp: k_imex_k1, k_imex_k2,
@@ -140,10 +153,9 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
       k_fixup<SYS, ZZ><<<1, FIX_BLOCK, 0, g->stream>>>(g->ga, g->V, U, g->fix, g->VS[0], g->VS[1], last,
                                                         ImexView{g->U[0], g->imex.P4, phase}, last);
     };
-    launch_sweeps<SYS, ZZ>(g);
+    launch_sweeps<SYS, ZZ>(g, irk);
     // dt from the speeds of the step's first sweeps, as in the RK steps
-    if (irk == 1) k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
-                                       sweep_blocks(g, 2));
+    if (irk == 1) k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, speed_max(g));
     if (g->timing) hipEventRecord(g->ev[4], g->stream);
     if (irk == 1) {
       // K2 = u0 (evolve.f90:232-233): its inversion; the repair also sets
@@ -177,8 +189,7 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
     if (g->timing) hipEventRecord(g->ev[0], g->stream);
     if (irk == 1) {
       if (g->timing) for (int i = 1; i < 4; i++) hipEventRecord(g->ev[i], g->stream);
-      k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, g->partial, sweep_blocks(g, 0), sweep_blocks(g, 1),
-                                       sweep_blocks(g, 2));
+      k_cfl<<<1, 1024, 0, g->stream>>>(g->ga, speed_max(g));
       if (g->timing) hipEventRecord(g->ev[4], g->stream);
       k_imex_k1<SYS, ZZ><<<nbu, UPDATE_BLOCK, 0, g->stream>>>(g->ga, g->V, g->U[0], Ust, g->fix);
       fixup(Ust, 0, 1);
@@ -187,7 +198,7 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
       fixup(Ust, 0, 2);
       return;
     }
-    launch_sweeps<SYS, ZZ>(g);
+    launch_sweeps<SYS, ZZ>(g, irk);
     if (g->timing) hipEventRecord(g->ev[4], g->stream);
 #define ECHO_IMEX_UPDATE(ST)                                                                        \
   k_update_imex<SYS, ZZ, ST><<<update_blocks(g), UPDATE_BLOCK, 0, g->stream>>>(                    \
@@ -203,18 +214,24 @@ static void enqueue_imex_stage_t(echo_grid* g, int irk) {
   }
 }
 
-static void enqueue_stage(echo_grid* g, int irk) {
+static void enqueue_fixup(echo_grid* g, int irk) {
+  dispatch_sys(g->cfg,
+               [&](auto sys, auto zz) { enqueue_fixup_t<decltype(sys)::value, decltype(zz)::value>(g, irk); });
+}
+
+// stage irk; fixup: with the repair of its failed cells (always, for IMEX)
+static void enqueue_stage(echo_grid* g, int irk, bool fixup = true) {
   dispatch_sys(g->cfg, [&](auto sys, auto zz) {
     constexpr int S = decltype(sys)::value;
     constexpr bool Z = decltype(zz)::value;
     if (g->cfg.nrk == 4) enqueue_imex_stage_t<S, Z>(g, irk);
-    else enqueue_stage_t<S, Z>(g, irk);
+    else enqueue_stage_t<S, Z>(g, irk, fixup);
   });
 }
 
 // one flux sweep (direction d = 0, 1, 2) with the current tile shape
 static void enqueue_flux(echo_grid* g, int d) {
-  dispatch_sys(g->cfg, [&](auto sys, auto zz) { launch_flux<decltype(sys)::value, decltype(zz)::value>(g, 1u << d); });
+  dispatch_sys(g->cfg, [&](auto sys, auto zz) { launch_flux<decltype(sys)::value, decltype(zz)::value>(g, 1u << d, 1); });
 }
 
 static int set_tile(echo_grid* g, int d, int ty) {
@@ -257,7 +274,7 @@ static int tune_grid(echo_grid* g, int reps, double* ms_out) {
 }
 
 static void enqueue_end_step(echo_grid* g) {
-  k_end_step<<<1, 64, 0, g->stream>>>(g->S, g->cfg.coordinates, g->cfg.viscosity ? 1 : 0);
+  k_end_step<<<1, 64, 0, g->stream>>>(g->S, g->cfg.coordinates, g->cfg.viscosity ? 1 : 0, g->cfg.nrk, g->ga.res);
 }
 
 static void enqueue_check(echo_grid* g) {
@@ -282,10 +299,10 @@ static void enqueue_dump_copy(echo_grid* g) {
                                                                         g->dump_buf[1], n);
 }
 
-static void enqueue_step(echo_grid* g) {
+static void enqueue_step(echo_grid* g, bool fixup = true) {
   enqueue_check(g);
   enqueue_dump_copy(g);
-  for (int irk = 1; irk <= g->cfg.nrk; irk++) enqueue_stage(g, irk);
+  for (int irk = 1; irk <= g->cfg.nrk; irk++) enqueue_stage(g, irk, fixup);
   enqueue_end_step(g);
 }
 
@@ -512,7 +529,7 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
     Eh.przero = pz;
     DevScalars S0{};
     S0.t = c.tmin; S0.timeold = c.tmin; S0.timeinterval = 0.; S0.g_cov_3_old = 0.;
-    S0.dt = c.maxdt; S0.tout = c.tmin + c.dtout; S0.dtout = c.dtout; S0.tmax = c.tmax;
+    S0.dt = S0.dts = c.maxdt; S0.tout = c.tmin + c.dtout; S0.dtout = c.dtout; S0.tmax = c.tmax;
     // resistive systems clean at the speed of light
     S0.glm_ch_old = c.mhd == 2 ? 1. : 0.5;
     S0.glm_ch = S0.glm_ch_old;
@@ -785,11 +802,15 @@ static int run_init(echo_grid* g) {
   return st;
 }
 
-// the run's crash state, with a message saying what crashed it
-static int read_crash(echo_grid* g) {
-  DevScalars S;
+static int read_scalars(echo_grid* g, DevScalars& S) {
   HIPCHECK(hipMemcpyAsync(&S, g->S, sizeof S, hipMemcpyDeviceToHost, g->stream));
   HIPCHECK(hipStreamSynchronize(g->stream));
+  g->iter = S.iter;
+  return 0;
+}
+
+// the run's crash state, with a message saying what crashed it
+static int crash_of(const echo_grid* g, const DevScalars& S) {
   if (!S.run_crashed) return 0;
   const int code = S.errcode > 0 ? S.errcode : ECHO_E_CRASHED;
   const int nx = g->cfg.nx, ny = g->cfg.ny;
@@ -809,6 +830,12 @@ static int read_crash(echo_grid* g) {
     default:
       return fail(code, "the run has crashed (error code %d), t=%.17g", S.errcode, S.t);
   }
+}
+
+static int read_crash(echo_grid* g) {
+  DevScalars S;
+  if (int e = read_scalars(g, S)) return e;
+  return crash_of(g, S);
 }
 
 int echo_rk_stage(echo_grid* g, int32_t irk) {
@@ -834,6 +861,22 @@ int echo_end_step(echo_grid* g) {
   HIPCHECK(hipGetLastError());
   g->next_stage = 1;
   return read_crash(g);
+}
+
+// n replays of the captured step, with or without the repairs
+static int launch_steps(echo_grid* g, int n, bool fixup) {
+  if (n <= 0) return 0;
+  if (!g->gexec) {
+    HIPCHECK(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
+    enqueue_step(g, fixup);
+    hipGraph_t graph;
+    HIPCHECK(hipStreamEndCapture(g->stream, &graph));
+    g->graph = graph;
+    HIPCHECK(hipGraphInstantiate(&g->gexec, graph, nullptr, nullptr, 0));
+  }
+  for (int s = 0; s < n; s++) HIPCHECK(hipGraphLaunch(g->gexec, g->stream));
+  HIPCHECK(hipGetLastError());
+  return 0;
 }
 
 int echo_steps(echo_grid* g, int32_t nsteps) {
@@ -869,16 +912,27 @@ int echo_steps(echo_grid* g, int32_t nsteps) {
     HIPCHECK(hipGetLastError());
     return read_crash(g);
   }
-  if (!g->gexec) {
-    HIPCHECK(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_step(g);
-    hipGraph_t graph;
-    HIPCHECK(hipStreamEndCapture(g->stream, &graph));
-    g->graph = graph;
-    HIPCHECK(hipGraphInstantiate(&g->gexec, graph, nullptr, nullptr, 0));
+  // Steps go without the repair's launches (3-4 us each, as long as a small
+  // grid's sweeps) until a step needs one: the kernels after a stage that left
+  // failed cells return at once (paused), the step is finished here with the
+  // repair, and from then on the grid's steps hold the repairs.  IMEX steps
+  // and the learned inversion always do.
+  int left = nsteps;
+  if (!g->repairs && g->cfg.nrk != 4 && !g->net) {
+    const int first = g->iter;
+    if (int e = launch_steps(g, left, false)) return e;
+    DevScalars S;
+    if (int e = read_scalars(g, S)) return e;
+    if (S.nfail == 0) return crash_of(g, S);
+    g->repairs = true;
+    drop_graph(g);
+    enqueue_fixup(g, S.fail_stage);
+    for (int irk = S.fail_stage + 1; irk <= g->cfg.nrk; irk++) enqueue_stage(g, irk);
+    enqueue_end_step(g);
+    HIPCHECK(hipGetLastError());
+    left -= S.iter - first + 1;
   }
-  for (int s = 0; s < nsteps; s++) HIPCHECK(hipGraphLaunch(g->gexec, g->stream));
-  HIPCHECK(hipGetLastError());
+  if (int e = launch_steps(g, left, true)) return e;
   return read_crash(g);
 }
 
@@ -888,6 +942,13 @@ int echo_get_scalars(echo_grid* g, double* s) {
   DevScalars S;
   HIPCHECK(hipMemcpyAsync(&S, g->S, sizeof S, hipMemcpyDeviceToHost, g->stream));
   HIPCHECK(hipStreamSynchronize(g->stream));
+  // inside a step (or one that crashed) dt and the cleaning speed are the
+  // running step's
+  if (g->next_stage > 1 || S.run_crashed) S.dt = S.dts;
+  if (g->next_stage > 1 && !g->ga.res) {
+    const double* f = S.aflux[g->next_stage - 2];
+    S.glm_ch_old = std::max(std::max(f[0], f[1]), f[2]);
+  }
   s[0] = S.t; s[1] = S.dt; s[2] = S.timeold; s[3] = S.timeinterval; s[4] = S.g_cov_3_old;
   s[5] = S.glm_ch_old; s[6] = S.tout; s[7] = S.iter; s[8] = S.run_crashed; s[9] = S.errcode;
   return 0;

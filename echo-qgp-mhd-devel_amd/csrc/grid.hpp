@@ -67,6 +67,8 @@ struct echo_grid {
   hipEvent_t ev[8] = {};
   double tms[4] = {0, 0, 0, 0};
   int next_stage = 1;
+  int iter = 0;               // steps taken, as of the last read of the scalars
+  bool repairs = false;       // the captured step holds the con2prim repairs (echo_steps)
   int tile[3] = {1, 1, 1};    // flux tile shape (TY) per sweep
   bool owns_scratch = true;   // F, L, partial (shared inside an ensemble)
   bool owns_stream = true;

@@ -19,9 +19,10 @@ namespace echo {
 
 struct DevScalars {
   double t, dt, timeold, timeinterval, g_cov_3_old, tout, glm_ch, glm_ch_old;
+  double dts;              // dt of the step in progress (dt: of the last one taken)
   double smooth_pressure, dtout, tmax;
   double temp_end;         // check_temp threshold (<= 0: no check)
-  double aflux[3];         // max(ap, am) at the last interface of each sweep
+  double aflux[4][3];      // per stage: max(ap, am) at the last interface of each sweep
   double check_max;        // max temperature (or energy density) of the last check
   long long nrepair;       // cells repaired by k_fixup since set-up
   long long nfallback;     // states the learned inversion in the step left to the plain solver
@@ -31,6 +32,8 @@ struct DevScalars {
   int temp_check;          // 1 once the check has stopped the run
   int crash_kind;          // what crashed the run: CRASH_* below
   int crash_cell;          // first cell (x fastest) whose repair failed
+  int paused;              // steps launched without k_fixup met failed cells (echo_steps)
+  int fail_stage;          // the stage that left failed cells
   int pad;
 };
 
@@ -68,6 +71,62 @@ struct GridArgs {
   int upd_tz;           // z rows per block of the cell updates (update_cell): 4 or 1
   DevScalars* S;
 };
+
+// The cleaning speed of stage irk: maxval(aflux) of the stage before
+// (evolve.f90:157-163), of the last step's last stage for the first; the
+// resistive systems clean at the speed of light.
+__device__ __forceinline__ double stage_ch(const GridArgs& a, int irk) {
+  if (a.res || irk <= 1) return a.S->glm_ch;
+  const double* f = a.S->aflux[irk - 2];
+  return dmax(dmax(f[0], f[1]), f[2]);
+}
+
+// The time step of evolve_dt (evolve.f90:723-764) with the clamps of
+// evolve.f90:179-188; amax: the largest of dd * speed over the sweeps' faces
+// (max over cells of dd * max(speeds) for a uniform grid).
+__device__ __forceinline__ double next_dt(const GridArgs& a, double amax) {
+  const DevScalars* S = a.S;
+  if (a.res) {
+    // resistive systems: the speed of light limits the step
+    const double g3 = make_metric(a.coordinates, S->t).g3;
+    amax = 0.;
+    if (a.nx > 1) amax = dmax(amax, a.ddx);
+    if (a.ny > 1) amax = dmax(amax, a.ddy);
+    if (a.nz > 1) amax = dmax(amax, a.ddz / sqrt(g3));
+  } else if (a.divclean) {
+    amax = 1.;   // evolve.f90:734-736
+  } else if (amax == 0) {
+    if (a.nx > 1) amax = dmax(amax, a.ddx);
+    if (a.ny > 1) amax = dmax(amax, a.ddy);
+    if (a.nz > 1) amax = dmax(amax, a.ddz);
+  }
+  double dt = a.cfl / amax;
+  dt = dmin(dt, a.maxdt);
+  dt = dmin(dt, S->tout - S->t);
+  if (fabs(S->t + S->dt - S->tout) < 1.e-9) dt = S->tout - S->t;
+  else if ((S->t + 2. * dt - S->tout) > 1.e-9) dt = (S->tout - S->t) / 2.;
+  return dt;
+}
+
+// per-block speed maxima of a stage's sweeps (nb[d] of direction d, one after
+// the other), and how many of them a block of the first update reduces by
+// itself; grids with more leave it to k_cfl
+struct SpeedMax {
+  const double* partial;
+  unsigned nb[3];
+};
+constexpr unsigned CFL_IN_UPDATE = 1024;
+
+// the largest dd * speed of the sweeps, by the threads tid of nt: each its share
+__device__ __forceinline__ double speed_share(const GridArgs& a, const SpeedMax& q, unsigned tid, unsigned nt) {
+  double m = 0.;
+  const unsigned n01 = q.nb[0] + q.nb[1], n = n01 + q.nb[2];
+  for (unsigned i = tid; i < n; i += nt)
+    m = dmax(m, (i < q.nb[0] ? a.ddx : i < n01 ? a.ddy : a.ddz) * q.partial[i]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = dmax(m, __shfl_xor(m, o, 64));
+  return m;
+}
 
 // IMEX-SSP3(4,3,3) scratch (resistive systems), nv components each, in
 // units of a rate (u = u0 - dt * rate).  Only the three E components carry
@@ -228,6 +287,7 @@ struct FluxBufs {
   double* partial[3];
   unsigned nb[3];
   int tx[3];
+  int irk;   // stage
 };
 
 template <int SYS>
@@ -242,7 +302,7 @@ struct FluxLds {
 template <int DIR, int REC, int SYS, bool ZZ>
 __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __restrict__ V, double* __restrict__ F,
                                            double* __restrict__ L, double* __restrict__ partial, unsigned block,
-                                           unsigned nblocks, int tx, FluxLds<SYS>& lds) {
+                                           unsigned nblocks, int tx, int irk, FluxLds<SYS>& lds) {
   constexpr bool VISC = SysT<SYS>::VISC;
   constexpr int NV = SysT<SYS>::NV;
   const int nx = a.nx, ny = a.ny, nz = a.nz;
@@ -478,7 +538,7 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
       // the normal B.  The reference sets wr(psi) = wl(psi) before taking
       // their difference, so the B update reduces to the average.
       constexpr int KB = SysT<SYS>::KB + DIR - 1, KG = SysT<SYS>::KG;
-      const double ch = S->glm_ch;
+      const double ch = stage_ch(a, irk);
       const double gl = wl[KG], gr = sw[KG][tr], bl = wl[KB], br = sw[KB][tr];
       const double g = 0.5 * (gl + gr) - (br - bl) * ch / 2, bm = 0.5 * (bl + br);
       wl[KG] = g; sw[KG][tr] = g;
@@ -521,7 +581,7 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
       double am = dmax(dmax(0., -vfl1), -vfr1);
       amax = dmax(ap, am);
       // aflux(dir) keeps the last interface of the sweep (work.f90:217,310,401)
-      if (f == nf - 1) a.S->aflux[DIR - 1] = amax;
+      if (f == nf - 1) a.S->aflux[irk - 1][DIR - 1] = amax;
       double a1 = (ap == 0.0 && am == 0.0) ? 1. : rcp_nr(ap + am);
       // resistive: B, E and psi with the speed of light (coordinate speed
       // 1 / sqrt(g_dir))
@@ -565,73 +625,33 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
                                                                       FluxBufs b) {
   __shared__ FluxLds<SYS> lds;
   if (a.S->temp_check) return;   // the run has stopped (check_temp)
+  if (a.S->nfail > 0) {          // failed cells to repair first (echo_steps)
+    if (threadIdx.x == 0) a.S->paused = 1;
+    return;
+  }
   unsigned i = blockIdx.x;
-  if (i < b.nb[0]) return flux_block<1, REC, SYS, ZZ>(a, V, b.F[0], b.L[0], b.partial[0], i, b.nb[0], b.tx[0], lds);
+  if (i < b.nb[0]) return flux_block<1, REC, SYS, ZZ>(a, V, b.F[0], b.L[0], b.partial[0], i, b.nb[0], b.tx[0], b.irk, lds);
   i -= b.nb[0];
   if (i < b.nb[1])
-    return flux_block<2, REC, SYS, ZZ>(a, V, b.F[1], b.L[1], b.partial[1], i, b.nb[1], b.tx[1], lds);
+    return flux_block<2, REC, SYS, ZZ>(a, V, b.F[1], b.L[1], b.partial[1], i, b.nb[1], b.tx[1], b.irk, lds);
   i -= b.nb[1];
-  flux_block<3, REC, SYS, ZZ>(a, V, b.F[2], b.L[2], b.partial[2], i, b.nb[2], b.tx[2], lds);
+  flux_block<3, REC, SYS, ZZ>(a, V, b.F[2], b.L[2], b.partial[2], i, b.nb[2], b.tx[2], b.irk, lds);
 }
 
 // ---------------------------------------------------------------------------
 // k_cfl: reduces the per-block speed maxima of the three sweeps and applies
-// evolve_dt (evolve.f90:723-764) and the clamps of evolve.f90:179-188.
-// One block.  partial holds nb0 + nb1 + nb2 values (the block counts of the
-// three sweeps, in this order, 0 for those of dimensions with one cell).
+// evolve_dt (next_dt).  One block.
 // ---------------------------------------------------------------------------
-static __global__ __launch_bounds__(1024) void k_cfl(GridArgs a, const double* __restrict__ partial,
-                                              int nb0, int nb1, int nb2) {
-  if (a.S->temp_check) return;
-  __shared__ double red[3][16];
-  double m[3] = {0., 0., 0.};
-  const int nb[3] = {nb0, nb1, nb2};
-  const bool act[3] = {a.nx > 1, a.ny > 1, a.nz > 1};
-  int off = 0;
-  for (int d = 0; d < 3; d++) {
-    if (act[d])
-      for (int i = threadIdx.x; i < nb[d]; i += blockDim.x) m[d] = dmax(m[d], partial[off + i]);
-    off += nb[d];
-  }
-  for (int d = 0; d < 3; d++) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m[d] = dmax(m[d], __shfl_xor(m[d], o, 64));
-    if ((threadIdx.x & 63) == 0) red[d][threadIdx.x >> 6] = m[d];
-  }
+static __global__ __launch_bounds__(1024) void k_cfl(GridArgs a, SpeedMax q) {
+  if (a.S->temp_check || a.S->paused) return;
+  __shared__ double red[16];
+  const double m = speed_share(a, q, threadIdx.x, 1024);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
-    const int nw = (blockDim.x + 63) / 64;
-    double mm[3];
-    for (int d = 0; d < 3; d++) {
-      mm[d] = red[d][0];
-      for (int w = 1; w < nw; w++) mm[d] = dmax(mm[d], red[d][w]);
-    }
-    // max over cells of dd*max(speeds) == dd*max(speeds) for a uniform grid
-    double amax = 0.;
-    if (a.nx > 1) amax = dmax(amax, a.ddx * mm[0]);
-    if (a.ny > 1) amax = dmax(amax, a.ddy * mm[1]);
-    if (a.nz > 1) amax = dmax(amax, a.ddz * mm[2]);
-    if (a.res) {
-      // resistive systems: the speed of light limits the step
-      const double g3 = make_metric(a.coordinates, a.S->t).g3;
-      amax = 0.;
-      if (a.nx > 1) amax = dmax(amax, a.ddx);
-      if (a.ny > 1) amax = dmax(amax, a.ddy);
-      if (a.nz > 1) amax = dmax(amax, a.ddz / sqrt(g3));
-    } else if (a.divclean) {
-      amax = 1.;   // evolve.f90:734-736
-    } else if (amax == 0) {
-      if (a.nx > 1) amax = dmax(amax, a.ddx);
-      if (a.ny > 1) amax = dmax(amax, a.ddy);
-      if (a.nz > 1) amax = dmax(amax, a.ddz);
-    }
-    DevScalars* S = a.S;
-    double dt_local = a.cfl / amax;
-    dt_local = dmin(dt_local, a.maxdt);
-    dt_local = dmin(dt_local, S->tout - S->t);
-    if (fabs(S->t + S->dt - S->tout) < 1.e-9) dt_local = S->tout - S->t;
-    else if ((S->t + 2. * dt_local - S->tout) > 1.e-9) dt_local = (S->tout - S->t) / 2.;
-    S->dt = dt_local;
+    double amax = red[0];
+    for (int w = 1; w < 16; w++) amax = dmax(amax, red[w]);
+    a.S->dts = next_dt(a, amax);
   }
 }
 
@@ -734,6 +754,15 @@ __device__ __forceinline__ void flux_div(const GridArgs& a, int x, int y, int z,
   }
 }
 
+// what a stage's update is told: the RK coefficients, the stage and whether it
+// is the last, and the sweeps' speeds (CFL)
+struct StageArgs {
+  double c1, c2;
+  SpeedMax speeds;
+  int irk, last;
+};
+static_assert(UPDATE_BLOCK / 64 == 4, "the update's block maximum");
+
 // Waves per SIMD that the update's registers allow for (192 x 192 x 128
 // cells).  Three (168 VGPRs) for viscous hydro and ideal MHD, without
 // spills: ideal MHD 0.195 ms instead of 0.208 at two on 160 x 150 x 70 cells,
@@ -760,24 +789,43 @@ constexpr int imex_update_waves() { return SYS == SYS_VRMHD ? (STAGE == 4 ? 2 : 
 // ALGO: the ideal-MHD inversion algorithm when the launch knows it (5), else 0
 // (read from the arguments).  With all algorithms in one kernel the ideal-MHD
 // update needs 178 VGPRs, two waves per SIMD; with algorithm 5 alone it runs
-// three without spills (0.195 instead of 0.288 ms a launch on 160 x 150 x 70
+// three (0.195 instead of 0.288 ms a launch on 160 x 150 x 70
 // cells, with the divisions taken out of algorithm 5).
-template <int SYS, bool ZZ, int ALGO>
+//
+// CFL: the update of a first stage on a small grid also forms dt from the
+// sweeps' block maxima (at most CFL_IN_UPDATE of them, up to four loads a
+// thread), which saves the launch of k_cfl: 5 of the 47 us of a 128 x 128 step.
+template <int SYS, bool ZZ, int ALGO, bool CFL>
 __global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
     GridArgs a, double* __restrict__ V, double* U0, const double* Ucur, double* Uout,
     const double* __restrict__ FX, const double* __restrict__ FY, const double* __restrict__ FZ,
     const double* __restrict__ LX, const double* __restrict__ LY, const double* __restrict__ LZ,
-    double* __restrict__ VS0, double* __restrict__ VS1, FixBufs fb, double c1,
-    double c2, int first_stage, int last_stage) {
+    double* __restrict__ VS0, double* __restrict__ VS1, FixBufs fb, StageArgs st) {
   constexpr bool VISC = SysT<SYS>::VISC;
   constexpr int NV = SysT<SYS>::NV;
+  DevScalars* S = a.S;
+  if (S->temp_check || S->paused) return;
+  const int first_stage = st.irk == 1, last_stage = st.last;
+  __shared__ double red[UPDATE_BLOCK / 64];
+  if constexpr (CFL) {
+    // dt from the sweeps' speeds, by every block for itself; it waits in LDS
+    const double m = speed_share(a, st.speeds, threadIdx.x, UPDATE_BLOCK);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const double dt = next_dt(a, dmax(dmax(red[0], red[1]), dmax(red[2], red[3])));
+      red[0] = dt;
+      if (blockIdx.x == 0) S->dts = dt;   // for the later stages
+    }
+    __syncthreads();
+  }
   int x, y, z;
   long long c;
-  if (!update_cell(a, x, y, z, c) || a.S->temp_check) return;
-  DevScalars* S = a.S;
+  if (!update_cell(a, x, y, z, c)) return;
   if (S->run_crashed) return;
   const Metric M = make_metric(a.coordinates, S->t);
   const long long N = a.N;
+  const double c1 = st.c1, c2 = st.c2;
   double du[NV];
   flux_div<NV>(a, x, y, z, FX, FY, FZ, du);
   double v[NV];
@@ -814,7 +862,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
 #pragma unroll
     for (int k = 0; k < NV; k++) du[k] = du[k] - src[k];
   }
-  const double dt = S->dt;
+  const double dt = CFL ? red[0] : S->dts;
   double u0[NV], uc[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) {
@@ -826,7 +874,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
     if (first_stage) {
       // evolve_glm_source(dt/2) before u0 = u (evolve.f90:196): the damped
       // psi is also the RK base of the later stages
-      const double ch = S->glm_ch;
+      const double ch = stage_ch(a, 1);
       double ef = exp(-(ch * ch) * a.glm_alpha * (dt / 2.));
       u0[KG] = u0[KG] * ef;
       uc[KG] = u0[KG];
@@ -839,7 +887,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
   if constexpr (SysT<SYS>::GLM) {
     constexpr int KG = SysT<SYS>::KG;
     if (last_stage) {   // evolve.f90:201
-      const double ch = S->glm_ch;
+      const double ch = stage_ch(a, st.irk);
       un[KG] = un[KG] * exp(-(ch * ch) * a.glm_alpha * (dt / 2.));
     }
   }
@@ -856,6 +904,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, update_waves<SYS>()) void k_update(
   if (e != 0) {
     atomicOr(&fb.failbits[c >> 5], 1u << (c & 31));
     atomicAdd(&S->nfail, 1);
+    S->fail_stage = st.irk;
   } else if (VISC && a.enable_smooth) {
     const double ps = S->smooth_pressure;
     if (v[KPR] < ps) {
@@ -962,7 +1011,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_imex_k1(GridArgs a, double* __
     us[k] = U0[(long long)k * N + c];
     v[k] = V[(long long)k * N + c];
   }
-  imex_solve<SYS, ZZ, false>(a, M, c, V, Ust, fb, us, v, IMEX_A * a.S->dt);
+  imex_solve<SYS, ZZ, false>(a, M, c, V, Ust, fb, us, v, IMEX_A * a.S->dts);
 }
 
 // the stiff rate of K1 (cell-local), P4 = b ds1, and K2 from
@@ -977,7 +1026,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK) void k_imex_k2(GridArgs a, double* __
   if (c >= a.N || a.S->temp_check || a.S->run_crashed) return;
   const long long N = a.N;
   const Metric M = make_metric(a.coordinates, a.S->t);
-  const double dt = a.S->dt;
+  const double dt = a.S->dts;
   double us[NV], v[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) {
@@ -1074,7 +1123,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, (imex_update_waves<SYS, STAGE>())) vo
 #pragma unroll
     for (int k = 0; k < 3; k++) ds[k] = -sst[k];
   }
-  const double dt = S->dt;
+  const double dt = S->dts;
   double u0[NV], un[NV];
 #pragma unroll
   for (int k = 0; k < NV; k++) u0[k] = __builtin_nontemporal_load(&U0[k * N + c]);
@@ -1124,7 +1173,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, (imex_update_waves<SYS, STAGE>())) vo
     for (int k = 0; k < NV; k++) __builtin_nontemporal_store(v[k], &V[(long long)k * N + c]);
   } else {
     if constexpr (T::GLM) {
-      const double ch = S->glm_ch;
+      const double ch = stage_ch(a, 4);
       un[T::KG] = un[T::KG] * exp(-(ch * ch) * a.glm_alpha * (dt / 2.));
     }
     __builtin_nontemporal_store(v[KPR], &fb.Pold[c]);
@@ -1218,7 +1267,7 @@ __device__ void repair_cell(const GridArgs& a, const Metric& M, long long c, dou
   // E its implicit solve found: earlier cells are read with that E (u_E =
   // sqrt(-g) E), later ones (not yet solved in the reference's loop) with E*.
   const int imex = iv.phase;
-  const double dt = S->dt;
+  const double dt = S->dts;
   bool repaired[6];
 #pragma unroll
   for (int j = 0; j < 6; j++) repaired[j] = nb[j] < c && fix_failed(fb.failbits, nb[j]);
@@ -1299,14 +1348,7 @@ __global__ __launch_bounds__(FIX_BLOCK) void k_fixup(GridArgs a, double* __restr
   __shared__ int scan[FIX_BLOCK + 1];
   if (t == 0) {
     sh_go = 0;
-    if (!S->temp_check) {
-      // glm_ch_old = maxval(aflux) of this stage; the next stage starts with
-      // glm_ch = glm_ch_old (evolve.f90:157-163)
-      // (resistive systems clean at the speed of light)
-      S->glm_ch_old = a.res ? 1. : dmax(dmax(S->aflux[0], S->aflux[1]), S->aflux[2]);
-      S->glm_ch = S->glm_ch_old;
-      sh_go = S->nfail > 0;
-    }
+    if (!S->temp_check) sh_go = S->nfail > 0;
   }
   __syncthreads();
   if (!sh_go) return;
@@ -1413,6 +1455,7 @@ __global__ __launch_bounds__(FIX_BLOCK) void k_fixup(GridArgs a, double* __restr
     if (fb.failbits[w]) fb.failbits[w] = 0u;
   if (t == 0) {
     S->nfail = 0;
+    S->paused = 0;
     S->nrepair += n;
   }
 }
@@ -1429,7 +1472,7 @@ static __global__ __launch_bounds__(UPDATE_BLOCK) void k_dump_copy(const DevScal
                                                                   const double* __restrict__ U,
                                                                   double* __restrict__ B0,
                                                                   double* __restrict__ B1, long long n) {
-  if (S->temp_check || S->run_crashed) return;
+  if (S->temp_check || S->run_crashed || S->nfail > 0) return;
   const long long i = (long long)blockIdx.x * UPDATE_BLOCK + threadIdx.x;
   if (i >= n) return;
   double* B = (S->iter & 1) ? B1 : B0;
@@ -1437,9 +1480,16 @@ static __global__ __launch_bounds__(UPDATE_BLOCK) void k_dump_copy(const DevScal
   B[n + i] = U[i];
 }
 
-static __global__ void k_end_step(DevScalars* S, int coordinates, int flip_vs) {
+static __global__ void k_end_step(DevScalars* S, int coordinates, int flip_vs, int nrk, int res) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (S->run_crashed || S->temp_check) return;
+  if (S->nfail > 0) S->paused = 1;   // failed cells to repair first (echo_steps)
+  if (S->run_crashed || S->temp_check || S->paused) return;
+  // glm_ch_old = maxval(aflux) of the last stage; the next step starts with
+  // glm_ch = glm_ch_old (evolve.f90:157-163)
+  const double* f = S->aflux[nrk - 1];
+  S->glm_ch_old = res ? 1. : dmax(dmax(f[0], f[1]), f[2]);
+  S->glm_ch = S->glm_ch_old;
+  S->dt = S->dts;
   S->timeold = S->t;
   S->t = S->t + S->dt;
   // g_cov_3_old = g_cov(3) of the step just taken (echo.f90:213)
@@ -1518,7 +1568,7 @@ static __global__ __launch_bounds__(CHECK_BLOCK) void k_check_temp(GridArgs a, c
                                                                    double* __restrict__ partial) {
   double m = 0.;
   const long long c = (long long)blockIdx.x * CHECK_BLOCK + threadIdx.x;
-  if (c < a.N && !a.S->temp_check) {
+  if (c < a.N && !a.S->temp_check && a.S->nfail == 0) {
     double en, temp, s;
     get_derived_data(a.eos, V[c], V[KPR * a.N + c], en, temp, s);
     m = a.S->freeze_type == 0 ? temp : en;
@@ -1537,7 +1587,7 @@ static __global__ __launch_bounds__(CHECK_BLOCK) void k_check_temp(GridArgs a, c
 
 static __global__ __launch_bounds__(1024) void k_check_decide(DevScalars* S, const double* __restrict__ partial,
                                                               int nb) {
-  if (S->temp_check) return;
+  if (S->temp_check || S->nfail > 0) return;
   __shared__ double red[16];
   double m = 0.;
   for (int i = threadIdx.x; i < nb; i += 1024) m = dmax(m, partial[i]);

@@ -684,14 +684,16 @@ __device__ __forceinline__ double f_comp(int k, const Metric& M, const SideState
 // ---------------------------------------------------------------------------
 struct MhdPar { double B2, SB2, S2, UU, D; };
 
-// x^(1/3) for x > 0, the start of the cubic's Newton iteration: the hardware's
-// single-precision logarithm and power (1e-6) and one Newton step on r^3 = x;
-// pow outside the range of a float
+// x^(1/3) for x >= 0, the start of the cubic's Newton iteration: x = m 2^3q,
+// the hardware's single-precision logarithm and power for m^(1/3) (1e-6) and
+// one Newton step on r^3 = m
 __device__ __forceinline__ double cbrt_start(double x) {
-  if (!(x > 1e-30 && x < 1e30)) return pow(x, 1.0 / 3.0);
-  const double r = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)x) * (1.0f / 3.0f));
+  if (x == 0.) return 0.;
+  const int q = __builtin_amdgcn_frexp_exp(x) / 3;
+  const double m = ldexp(x, -3 * q);
+  const double r = (double)__builtin_amdgcn_exp2f(__builtin_amdgcn_logf((float)m) * (1.0f / 3.0f));
   const double r2 = r * r;
-  return r - quot(r2 * r - x, 3. * r2);
+  return ldexp(r - quot(r2 * r - m, 3. * r2), q);
 }
 
 template <bool IDEALGAS>
