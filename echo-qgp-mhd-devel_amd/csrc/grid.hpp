@@ -69,7 +69,8 @@ struct echo_grid {
   int next_stage = 1;
   int iter = 0;               // steps taken, as of the last read of the scalars
   bool repairs = false;       // the captured step holds the con2prim repairs (echo_steps)
-  int tile[3] = {1, 1, 1};    // flux tile shape (TY) per sweep
+  int tile[3] = {1, 1, 1};    // flux tile shape per sweep (echo_set_tile)
+  bool tile_set = false;      // set or tuned; until then flux_tx chooses
   bool owns_scratch = true;   // F, L, partial (shared inside an ensemble)
   bool owns_stream = true;
   long long partial_cap = 0;  // doubles in partial

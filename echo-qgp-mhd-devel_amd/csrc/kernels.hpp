@@ -264,12 +264,14 @@ constexpr int flux_group() {
   return SysT<SYS>::NV == 5 || SYS == SYS_MHDGLM ? 5 : 4;
 }
 
-// Launch bounds: three waves per SIMD (at most 168 VGPRs); 49 KB of LDS per
-// block for NV = 12 (three blocks per CU).  The viscous resistive system
-// (NV = 19, 64 KB per block) fits two blocks per CU, two waves per SIMD, and
-// is bounded for that.
+// Launch bounds: three waves per SIMD (at most 168 VGPRs), which the viscous
+// resistive system (NV = 19, 160 VGPRs, 51 KB of LDS per block) takes; the
+// smaller systems run four (114 VGPRs, 37 KB for NV = 12), hydro six.
+// With a second staging buffer (one barrier per group instead of two) the
+// LDS allowed two and three: 0.62 instead of 0.54 ms a sweep for NV = 19,
+// 0.40 instead of 0.36 for NV = 12, on 192 x 192 x 128 cells.
 template <int SYS>
-constexpr int flux_waves() { return SysT<SYS>::NV > 12 ? 2 : 3; }
+constexpr int flux_waves() { return SysT<SYS>::NV > 5 ? 3 : 6; }
 
 // barrier of the block that orders its LDS accesses only: loads from memory
 // stay in flight across it
@@ -293,9 +295,9 @@ struct FluxBufs {
 template <int SYS>
 struct FluxLds {
   static constexpr int NI = SysT<SYS>::NV + (SysT<SYS>::VISC ? 4 : 0);
-  static constexpr int GS = flux_group<SYS>(), NG = (NI + GS - 1) / GS, NBUF = NG > 1 ? 2 : 1;
+  static constexpr int GS = flux_group<SYS>(), NG = (NI + GS - 1) / GS;
   double sw[SysT<SYS>::NV][FLUX_BLOCK];
-  double st[NBUF][GS][FLUX_STAGE];
+  double st[GS][FLUX_STAGE];
   double red[FLUX_BLOCK / 64];
 };
 
@@ -353,7 +355,7 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
   const DevScalars* S = a.S;
   const Metric M = make_metric(a.coordinates, S->t);
   // Staging.  The tile's cells with two more at either end of the sweep pass
-  // through LDS, GS components at a time (st, two buffers): every value is
+  // through LDS, GS components at a time (st): every value is
   // loaded from memory once per tile, the loads of the next group are in
   // flight while this one is reconstructed, and the five cells of a thread's
   // stencil are LDS reads.  sw: the lower states.  Thread t reads the lower
@@ -363,7 +365,7 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
   // gamma v^i), reconstructed for deriv (evolve.f90:324-331, 371-374); it is
   // formed once per staged cell.
   constexpr int NU = VISC ? 4 : 0, NI = NV + NU;
-  constexpr int GS = FluxLds<SYS>::GS, NG = FluxLds<SYS>::NG, NBUF = FluxLds<SYS>::NBUF;
+  constexpr int GS = FluxLds<SYS>::GS, NG = FluxLds<SYS>::NG;
   static_assert(!VISC || (GS == 4 && NG >= 4), "the Lorentz velocity's lower states wait in the last group's slots");
   auto& sw = lds.sw;
   auto& st = lds.st;
@@ -441,10 +443,10 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
     if (VISC && g == 0) {
       auto lorentz = [&](const double* v, unsigned p) {
         const double gl = rsqrt_nr(1. - v[0] * v[0] - v[1] * v[1] - M.g3 * (v[2] * v[2]));
-        st[0][0][p] = gl;
-        st[0][1][p] = gl * v[0];
-        st[0][2][p] = gl * v[1];
-        st[0][3][p] = gl * v[2];
+        st[0][p] = gl;
+        st[1][p] = gl * v[0];
+        st[2][p] = gl * v[1];
+        st[3][p] = gl * v[2];
       };
       lorentz(va, t);
       if (second) lorentz(vb, FLUX_BLOCK + t);
@@ -452,13 +454,13 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
 #pragma unroll
       for (int q = 0; q < GS; q++) {
         if (g * GS + q >= NI) break;
-        st[g % NBUF][q][t] = ra[q];
+        st[q][t] = ra[q];
       }
       if (second) {
 #pragma unroll
         for (int q = 0; q < GS; q++) {
           if (g * GS + q >= NI) break;
-          st[g % NBUF][q][FLUX_BLOCK + t] = rb[q];
+          st[q][FLUX_BLOCK + t] = rb[q];
         }
       }
     }
@@ -479,14 +481,14 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
       if (it >= NI) break;
       double s[5], h, l;
 #pragma unroll
-      for (int j = 0; j < 5; j++) s[j] = st[g % NBUF][q][ps[j]];
+      for (int j = 0; j < 5; j++) s[j] = st[q][ps[j]];
       rec_cell<REC>(s, h, l);
       // h is used below only by the threads that own an interface: without
       // this the compiler moves its arithmetic there and keeps the inputs
       asm volatile("" : "+v"(h));
       if (k < 0) {
         wu[it] = h;
-        sw[NV - 4 + it][t] = l;   // rewritten two barriers after it was read
+        sw[NV - 4 + it][t] = l;   // rewritten by the last group, barriers after it was read
         continue;
       }
       wl[k] = h;
@@ -496,12 +498,13 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
         if (k == SysT<SYS>::KE + DIR - 1) dEface = s[3] - s[2];
       }
     }
+    if (g + 1 < NG) block_sync_lds();   // the group's cells are read
   }
   block_sync_lds();
-  // the left states of the first NPK components wait in the staging buffers
-  constexpr int NPK = NV < NBUF * GS * FLUX_STAGE / FLUX_BLOCK ? NV : NBUF * GS * FLUX_STAGE / FLUX_BLOCK;
+  // the left states of the first NPK components wait in the staging buffer
+  constexpr int NPK = NV < GS * FLUX_STAGE / FLUX_BLOCK ? NV : GS * FLUX_STAGE / FLUX_BLOCK;
   static_assert(NPK > KPR, "the fluid's left states are parked");
-  double* pk = &st[0][0][0] + t;
+  double* pk = &st[0][0] + t;
   double amax = 0.;
   if (owns) {
     double wr[5];

@@ -314,12 +314,14 @@ int echo_cons2prim_batch(echo_grid *g, const double *u, double *v, int32_t *stat
                          int64_t n);
 
 /* Tile shape of the flux sweeps and its autotuner (no counterpart in the
- * reference, whose sweeps are pencil loops, evolve.f90:302-685).  A y or z
- * sweep with `rows` = 2 or 4 runs blocks of 256/rows faces along x by `rows`
- * faces along the sweep (WENO5 and PPM4); results are identical for every
- * shape.  echo_tune times each shape on the current state (reps launches
- * each) and keeps the fastest; ms (optional, 9 doubles): per-launch times,
- * [3*sweep + {0,1,2}] for rows {1,2,4}. */
+ * reference, whose sweeps are pencil loops, evolve.f90:302-685).  The blocks
+ * of a y or z sweep are 16 cells along x by 16 along the sweep with rows = 1,
+ * 32 by 8 with rows = 2, 8 by 32 with rows = 4 (WENO5 and PPM4); results are
+ * identical for every shape.  Until a shape is set or tuned the sweeps take
+ * one of the first two by the grid's size.  echo_tune times each shape
+ * on the current state (reps launches each) and keeps the fastest; ms
+ * (optional, 9 doubles): per-launch times, [3*sweep + {0,1,2}] for rows
+ * {1,2,4}. */
 int echo_set_tile(echo_grid *g, int32_t sweep, int32_t rows);
 int echo_get_tile(const echo_grid *g, int32_t *rows);
 int echo_tune(echo_grid *g, int32_t reps, double *ms);
