@@ -98,7 +98,7 @@ static bool tiles_supported(const echo_config& c) { return c.recal == REC_WENO5 
 // launch blocks of the cell updates (update_cell), padded for xcd_block
 static unsigned update_blocks(const echo_grid* g) {
   if (g->ga.upd_tz == 1) return nblocks_xcd(g->N, UPDATE_BLOCK);
-  const long long t = (long long)((g->cfg.nx + UPD_TX - 1) / UPD_TX) * g->cfg.ny * ((g->cfg.nz + UPD_TZ - 1) / UPD_TZ);
+  const long long t = ((long long)g->cfg.nx * g->cfg.ny + UPD_TX - 1) / UPD_TX * ((g->cfg.nz + UPD_TZ - 1) / UPD_TZ);
   return (unsigned)((t + NXCD - 1) / NXCD * NXCD);
 }
 
@@ -581,9 +581,10 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
   a.sch = c.sigma_chi / 0.197326;
   a.ext_c2p = 0;
   // z-row tiles for the MHD systems, whose updates read the most face data
-  // (measured: viscous resistive step 2.1% faster, ideal MHD 1% faster,
-  // viscous hydro 0.6% slower than cells in storage order)
-  a.upd_tz = (c.mhd && c.nz >= UPD_TZ && c.nx >= UPD_TX) ? UPD_TZ : 1;
+  // (measured: viscous resistive step 2.1% faster, ideal MHD 1% faster than
+  // with cells in storage order; viscous hydro 0.91 ms a launch in storage
+  // order, 0.92 in tiles)
+  a.upd_tz = (c.mhd && c.nz >= UPD_TZ) ? UPD_TZ : 1;
   a.S = g->S;
   if (!share_scratch && hipMemset(g->fix.failbits, 0, sizeof(unsigned) * (size_t)fix_words(g->N)) != hipSuccess) {
     release(g);

@@ -174,15 +174,17 @@ __device__ __forceinline__ long long xcd_block(unsigned b, unsigned nb) {
 }
 
 // Cell of a cell-update thread (k_update, k_update_imex).  With upd_tz = 4 a
-// block is a tile of 64 x-consecutive cells by 4 z-consecutive rows (one
-// wave per row), tiles ordered x chunk fastest, then y, then z.  A cell
-// reads the z faces below and above it, and the face between two rows of a
-// tile is read by both rows within the block: the face arrays of the z
-// sweep are fetched about once, not once per side (with the cells in
-// storage order the row above comes nx * ny cells later, long after the
-// face has left the XCD's L2).  MHD grids with at least 64 cells in x and
-// 4 in z use the tiles; with upd_tz = 1 the cells go in storage order,
-// UPDATE_BLOCK per block.
+// block is a tile of 64 consecutive cells of a z plane (rows of x one after
+// the other) by 4 z-consecutive planes (one wave per plane), tiles ordered
+// along the plane, then z.  A cell reads the z faces below and above it, and
+// the face between two planes of a tile is read by both within the block: the
+// face arrays of the z sweep are fetched about once, not once per side (with
+// the cells in storage order the plane above comes nx * ny cells later, long
+// after the face has left the XCD's L2).  Taking the plane's cells in
+// sequence leaves no idle lanes at row ends (131 x 117 x 75 cells, viscous
+// resistive: 0.413 ms a launch, 0.481 with tiles of 64 cells of one row).
+// MHD grids with at least 4 cells in z use the tiles; with upd_tz = 1 the
+// cells go in storage order, UPDATE_BLOCK per block.
 // Returns false for the padding threads of the launch.
 constexpr int UPD_TX = 64, UPD_TZ = 4;
 static_assert(UPDATE_BLOCK == UPD_TX * UPD_TZ && UPD_TX == 64, "a tile row is one wave of 64 lanes");
@@ -198,13 +200,13 @@ __device__ __forceinline__ bool update_cell(const GridArgs& a, int& x, int& y, i
     y = (int)(r - (unsigned)z * ny);
     return true;
   }
-  const unsigned nxc = (nx + UPD_TX - 1) / UPD_TX;
-  const unsigned r = b / nxc, rz = r / ny;
-  x = (int)((b - r * nxc) * UPD_TX + (threadIdx.x & (UPD_TX - 1)));
-  y = (int)(r - rz * ny);
+  const unsigned plane = nx * ny, np = (plane + UPD_TX - 1) / UPD_TX;
+  const unsigned rz = b / np, i = (b - rz * np) * UPD_TX + (threadIdx.x & (UPD_TX - 1));
+  y = (int)(i / nx);
+  x = (int)(i - (unsigned)y * nx);
   z = (int)(rz * UPD_TZ + (threadIdx.x >> 6));
-  if (x >= a.nx || z >= a.nz) return false;
-  c = x + (long long)nx * (y + ny * (unsigned)z);
+  if (i >= plane || z >= a.nz) return false;
+  c = i + (long long)plane * z;
   return true;
 }
 
@@ -1141,13 +1143,13 @@ __global__ __launch_bounds__(UPDATE_BLOCK, (imex_update_waves<SYS, STAGE>())) vo
       const double s = ds[ke];
       if constexpr (STAGE == 2) {
         ib.P4[o] = ib.P4[o] + (du[k] / 4. + IMEX_H * s);
-        ib.ACC[o] = du[k] / 6. + s / 6.;
+        ib.ACC[o] = (du[k] + s) * (1. / 6.);
         un[k] = __builtin_fma(-dt, du[k] + (1. - IMEX_A) * s, u0[k]);
       } else if constexpr (STAGE == 3) {
         un[k] = __builtin_fma(-dt, ib.P4[o] + du[k] / 4. + IMEX_D * s, u0[k]);
-        ib.ACC[o] = ib.ACC[o] + (du[k] / 6. + s / 6.);
+        ib.ACC[o] = ib.ACC[o] + (du[k] + s) * (1. / 6.);
       } else {
-        un[k] = __builtin_fma(-dt, ib.ACC[o] + du[k] * 2. / 3. + s * 2. / 3., u0[k]);
+        un[k] = __builtin_fma(-dt, ib.ACC[o] + (du[k] + s) * (2. / 3.), u0[k]);
       }
     } else {
       if constexpr (STAGE == 2) {
@@ -1158,7 +1160,7 @@ __global__ __launch_bounds__(UPDATE_BLOCK, (imex_update_waves<SYS, STAGE>())) vo
         ib.P4[o] = r3;
         un[k] = __builtin_fma(-dt, r3, u0[k]);
       } else {
-        un[k] = __builtin_fma(-dt, ib.P4[o] * (2. / 3.) + du[k] * 2. / 3., u0[k]);
+        un[k] = __builtin_fma(-dt, (ib.P4[o] + du[k]) * (2. / 3.), u0[k]);
       }
     }
   }
