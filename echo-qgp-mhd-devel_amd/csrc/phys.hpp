@@ -188,6 +188,32 @@ __host__ __device__ __forceinline__ int eos_pressure(const Eos& E, double rh, do
   return 0;
 }
 
+// eos_pressure inside an inversion, whose Newton iterates mostly stay in one
+// bracket of the table: the bracket of the last lookup is kept, and while en
+// lies in it (e1 < en <= e2: the same index) there is nothing to look up.  A
+// lookup is three dependent loads (bin start, entry, row), and an inversion
+// made one per iterate.
+struct EosBracket { double e1 = __builtin_inf(), e2 = 0., p1 = 0., slope = 0.; };
+
+__device__ __forceinline__ int eos_pressure_near(const Eos& E, double rh, double en, EosBracket& b, double& pr,
+                                                 double& dprdrh, double& dprden) {
+  if (E.eqstate != 3) return eos_pressure(E, rh, en, pr, dprdrh, dprden);
+  if (!(en > b.e1 && en <= b.e2)) {
+    if (en < E.te[0]) return 123;
+    if (en > E.te[E.n - 1]) return 124;
+    const int l = bracket_e(E, en);
+    const double p2 = E.tp[l];
+    b.p1 = E.tp[l - 1];
+    b.e2 = E.te[l];
+    b.e1 = E.te[l - 1];
+    b.slope = quot(p2 - b.p1, b.e2 - b.e1);
+  }
+  dprden = b.slope;
+  pr = b.p1 + dprden * (en - b.e1);
+  dprdrh = 0;
+  return 0;
+}
+
 // eos_energy_ana (eos.f90:1108-1200) / get_energy (eos.f90:468-523)
 __host__ __device__ __forceinline__ int eos_energy(const Eos& E, double rh, double pr, double& en) {
   if (E.eqstate != 3) {
@@ -1111,6 +1137,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
   // before the first successful call the reference reads uninitialised
   // locals there.  They start at 0 here.
   double pr, w = 0., iw = 0., v2 = 0., glf, rh = 0., en, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
+  EosBracket br;
   if constexpr (!VISC) {
     pr = v[KPR];
     for (int iter = 1; iter <= 100; iter++) {
@@ -1125,7 +1152,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
         rh = d / glf;
         drh = rh * v2 * glf / (en + pr);
       }
-      errcode = eos_pressure(E, rh, en, pr_eos, dprdrh, dprden);
+      errcode = eos_pressure_near(E, rh, en, br, pr_eos, dprdrh, dprden);
       f = pr_eos - pr;
       df = dprdrh * drh + dprden * v2 - 1.;
       dpr = -quot(f, df);
@@ -1175,7 +1202,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
           rh = d / glf;
           drh = rh * v2 * glf / (en + pr);
         }
-        errcode = eos_pressure(E, rh, en, pr_eos, dprdrh, dprden);
+        errcode = eos_pressure_near(E, rh, en, br, pr_eos, dprdrh, dprden);
         f = pr_eos - pr;
         df = dprdrh * drh + dprden * v2 - 1.;
         dpr = -quot(f, df);
