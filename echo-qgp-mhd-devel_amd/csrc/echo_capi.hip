@@ -543,6 +543,7 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
     Eh.przero = pz;
     DevScalars S0{};
     S0.t = c.tmin; S0.timeold = c.tmin; S0.timeinterval = 0.; S0.g_cov_3_old = 0.;
+    set_metric(S0, c.coordinates);
     S0.dt = S0.dts = c.maxdt; S0.tout = c.tmin + c.dtout; S0.dtout = c.dtout; S0.tmax = c.tmax;
     // resistive systems clean at the speed of light
     S0.glm_ch_old = c.mhd == 2 ? 1. : 0.5;
@@ -1168,7 +1169,9 @@ int echo_restart(echo_grid* g, const char* path, int32_t* iout, double* thyp) {
   HIPCHECK(hipMemcpyAsync(&S, g->S, sizeof S, hipMemcpyDeviceToHost, g->stream));
   HIPCHECK(hipStreamSynchronize(g->stream));
   // out_restart, then system_metric and tout = t + dtout (echo.f90:164-172)
-  S.t = t; S.timeold = timeold; S.timeinterval = timeinterval; S.g_cov_3_old = g3old;
+  S.t = t;
+  set_metric(S, g->cfg.coordinates);
+  S.timeold = timeold; S.timeinterval = timeinterval; S.g_cov_3_old = g3old;
   S.tout = t + S.dtout;
   S.run_crashed = 0; S.errcode = 0; S.temp_check = 0;
   S.crash_kind = CRASH_NONE; S.crash_cell = 0x7fffffff;

@@ -131,7 +131,7 @@ inline void drop_graph(echo_grid* g) {
 namespace echo {
 
 inline unsigned nblocks(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
-// block count padded to a multiple of the XCD count (see xcd_block)
+// block count padded to a multiple of the XCD count
 inline unsigned nblocks_xcd(long long n, int bs) {
   unsigned nb = nblocks(n, bs);
   return (nb + NXCD - 1) / NXCD * NXCD;

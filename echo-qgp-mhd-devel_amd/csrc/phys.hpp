@@ -96,6 +96,9 @@ __device__ __forceinline__ double rsqrt_nr(double x) {
   return x == 0.0 ? __builtin_inf() : y;
 }
 
+// sqrt(x) for 0 <= x in the normal range, x times its reciprocal root
+__device__ __forceinline__ double sqrt_nr(double x) { return x == 0.0 ? 0.0 : x * rsqrt_nr(x); }
+
 // x / d for finite d != 0 in the normal range, by the reciprocal on the device
 // (four instructions and a product instead of the IEEE sequence; within about
 // an ulp of the quotient)
@@ -599,7 +602,7 @@ __device__ __forceinline__ void side_speeds(const Metric& M, const SideState& s,
   double a2 = s.cs2 + ca2 - s.cs2 * ca2;
   double den = rcp_nr(1. - s.v2 * a2);
   double vf1 = den * (1. - a2) * s.vdir;
-  double vf2 = den * sqrt(a2 * (1. - s.v2) * ((1. - s.v2 * a2) * igdir - (1. - a2) * (s.vdir * s.vdir)));
+  double vf2 = den * sqrt_nr(a2 * (1. - s.v2) * ((1. - s.v2 * a2) * igdir - (1. - a2) * (s.vdir * s.vdir)));
   lp = vf1 + vf2;
   lm = vf1 - vf2;
 }
