@@ -112,8 +112,8 @@ __device__ __forceinline__ f32x4 mfma16(h16x4 a, h16x4 b, f32x4 c) {
 // logarithms, the square root and the two quotients that follow only feed
 // half-precision inputs and are evaluated in FP32 with the hardware log2,
 // sqrt and reciprocal (the FP64 library calls took a third of the kernel).
-__device__ __forceinline__ void features(const double* u, double g33, float* x) {
-  const double S2 = u[1] * u[1] + u[2] * u[2] + u[3] * u[3] / g33;
+__device__ __forceinline__ void features(const double* u, double g33, double ig33, float* x) {
+  const double S2 = u[1] * u[1] + u[2] * u[2] + u[3] * u[3] * ig33;
   const double B2 = u[5] * u[5] + u[6] * u[6] + u[7] * u[7] * g33;
   const double SB = u[1] * u[5] + u[2] * u[6] + u[3] * u[7];
   const double iU = rcp_nr(u[4]);
@@ -142,7 +142,7 @@ __device__ __forceinline__ void features(const double* u, double g33, float* x) 
 __device__ __forceinline__ double w_baseline(double S2, double B2, double U) {
   const double Up = dmax(U - 0.5 * B2, 1e-3 * U);
   const double disc = dmax(4.0 * Up * Up - 3.0 * S2, 0.0);
-  const double p0 = dmax((-Up + sqrt(disc)) / 3.0, 1e-3 * Up);
+  const double p0 = dmax((1.0 / 3.0) * (sqrt_nr(disc) - Up), 1e-3 * Up);
   return Up + p0;
 }
 
@@ -166,52 +166,72 @@ __device__ __forceinline__ void targets(const double* u, const double* v, double
 // rtsafe on the momentum equation in x = v^2.  The momentum equation is
 // linear in x, so x(W) = (S^2 + (2W + B^2)(S.B)^2/W^2) / (W + B^2)^2 exactly,
 // and the refinement is Newton on f(W) = c3(x) W^3 + c2(x) W^2 - (S.B)^2/2
-// alone (c3 = (3 + x)/4, c2 = B^2 (1 + x)/2 - U), from the network's W.
-__device__ __forceinline__ void e3p_w(double W, double S2, double B2, double SB2, double U, double& f,
-                                      double& df, double& x, double& dxdw) {
-  const double iw = rcp_nr(W);
-  const double wb = W + B2;
-  const double iwb = rcp_nr(wb);
-  const double sbw2 = SB2 * iw * iw;
-  x = (S2 + (2.0 * W + B2) * sbw2) * iwb * iwb;
-  dxdw = (2.0 * sbw2 - 2.0 * (2.0 * W + B2) * sbw2 * iw) * iwb * iwb - 2.0 * x * iwb;
-  const double c3 = 0.25 * (3.0 + x);
-  const double c2 = 0.5 * B2 * (1.0 + x) - U;
-  f = (c3 * W + c2) * W * W - 0.5 * SB2;
-  df = W * (3.0 * c3 * W + 2.0 * c2) + W * W * (0.25 * W + 0.5 * B2) * dxdw;
+// alone (c3 = (3 + x)/4, c2 = B^2 (1 + x)/2 - U), from the network's W.  With
+// y = x W^2 = (S^2 W^2 + (2W + B^2)(S.B)^2) / (W + B^2)^2 it reads
+//   f = (3W/4 + B^2/2 - U) W^2 + (W/4 + B^2/2) y - (S.B)^2/2,
+// which takes one reciprocal an iterate.
+struct E3pInv {
+  double S2, B2, SB, SB2;
+  double h2;   // B^2 / 2
+  double b;    // B^2/2 - U
+};
+
+__device__ __forceinline__ E3pInv e3p_inv(const double* u, double g33, double ig33) {
+  E3pInv q;
+  q.S2 = u[1] * u[1] + u[2] * u[2] + u[3] * u[3] * ig33;
+  q.B2 = u[5] * u[5] + u[6] * u[6] + u[7] * u[7] * g33;
+  q.SB = u[1] * u[5] + u[2] * u[6] + u[3] * u[7];
+  q.SB2 = q.SB * q.SB;
+  q.h2 = 0.5 * q.B2;
+  q.b = q.h2 - u[4];
+  return q;
+}
+
+__device__ __forceinline__ void e3p_w(double W, const E3pInv& q, double& f, double& df, double& y,
+                                      double& dy, double& iwb) {
+  iwb = rcp_nr(W + q.B2);
+  const double sw = q.S2 * W + q.SB2;
+  y = (W * (sw + q.SB2) + q.B2 * q.SB2) * (iwb * iwb);
+  dy = 2.0 * iwb * (sw * iwb - y);
+  const double a = 0.25 * W + q.h2;
+  f = W * W * (0.75 * W + q.b) + (a * y - 0.5 * q.SB2);
+  df = W * (2.25 * W + 2.0 * q.b) + (a * dy + 0.25 * y);
 }
 
 // Newton refinement of the network's W (y1 = 25 log(W/W0)) and the residual
 // gate: accepted when the Newton correction dW at the final W is below
 // tol * W, the change it implies in 1 - v^2 is below tol * (1 - v^2), and
 // 0 <= v^2 < 1.  u: the de-densitised state; writes the 8 primitives.
-__device__ __forceinline__ bool refine(const double* u, float y1, double g33, int iters, double tol,
-                                       double* v) {
-  const double S2 = u[1] * u[1] + u[2] * u[2] + u[3] * u[3] / g33;
-  const double B2 = u[5] * u[5] + u[6] * u[6] + u[7] * u[7] * g33;
-  const double SB = u[1] * u[5] + u[2] * u[6] + u[3] * u[7];
-  const double SB2 = SB * SB, U = u[4];
+__device__ __forceinline__ bool refine(const double* u, float y1, double g33, double ig33, int iters,
+                                       double tol, double* v) {
+  const E3pInv q = e3p_inv(u, g33, ig33);
   // the guess needs no more than float precision: exp2 on the hardware
-  double W = w_baseline(S2, B2, U) * (double)__builtin_amdgcn_exp2f(y1 * (1.44269504f / 25.0f));
-  double f, df, x, dxdw;
+  double W = w_baseline(q.S2, q.B2, u[4]) * (double)__builtin_amdgcn_exp2f(y1 * (1.44269504f / 25.0f));
+  double f, df, y, dy, iwb;
   for (int it = 0; it < iters; it++) {
-    e3p_w(W, S2, B2, SB2, U, f, df, x, dxdw);
+    e3p_w(W, q, f, df, y, dy, iwb);
     W -= f * rcp_nr(df);
   }
-  e3p_w(W, S2, B2, SB2, U, f, df, x, dxdw);
+  e3p_w(W, q, f, df, y, dy, iwb);
   const double dW = f * rcp_nr(df);
+  const double iw = rcp_nr(W);
+  // 1 - x from the squares' difference: x as a quotient would carry its
+  // roundings into the cancellation
+  const double wb = W + q.B2, xs = (2.0 * W + q.B2) * (q.SB2 * iw * iw);
+  const double x = (q.S2 + xs) * iwb * iwb;
+  const double omx = (__builtin_fma(wb, wb, -q.S2) - xs) * iwb * iwb;
+  const double dxdw = (dy * iw - 2.0 * x) * iw;
   // the correction's effect on W and on 1 - v^2 (p and rho scale with it)
   const bool ok = (W > 0.0) && (x >= 0.0) && (x < 1.0) && (fabs(dW) <= tol * W) &&
-                  (fabs(dxdw * dW) <= tol * (1.0 - x));
+                  (omx > 0.0) && (fabs(dxdw * dW) <= tol * omx);
   if (!ok) return false;
   // primitives as at the end of algorithm 5 (system.f90:990-998)
-  const double vb = SB * rcp_nr(W);
-  const double iwb = rcp_nr(W + B2);
-  v[0] = u[0] * sqrt(1.0 - x);
-  v[4] = 0.25 * (1.0 - x) * W;
+  const double vb = q.SB * iw;
+  v[0] = u[0] * sqrt_nr(omx);
+  v[4] = 0.25 * omx * W;
   v[1] = (u[1] + vb * u[5]) * iwb;
   v[2] = (u[2] + vb * u[6]) * iwb;
-  v[3] = (u[3] / g33 + vb * u[7]) * iwb;
+  v[3] = (u[3] * ig33 + vb * u[7]) * iwb;
   v[5] = u[5];
   v[6] = u[6];
   v[7] = u[7];
@@ -235,9 +255,18 @@ struct C2pArgs {
   int in_step;            // inside a grid's step: nothing to do once the run stopped
 };
 
+// What bounds it: the SIMDs' issue.  Counted over 2^24 states, vector
+// instructions hold a SIMD for 68 % of the cycles and MFMA for another 32 %, and
+// the kernel takes what instructions are taken out of it: .67 ms with two
+// reciprocals an iterate, divisions and addresses per lane; .60 ms (2.2 GB, 3.6
+// TB/s; a streaming copy's time would be .35) with the one-reciprocal residual
+// (e3p_w) and a wave's tile at a scalar base.  States are read and written
+// once, past the caches (nontemporal, .02 ms).
 // Launch bounds (BLOCK, 3): three waves per SIMD (at most 168 VGPRs; the
 // inference variant takes 160 with no spills).  With two, the FP64 Newton
-// steps and the MFMA chains stall with too little to switch to.
+// steps and the MFMA chains stall with too little to switch to; four (blocks
+// of 512 and half the states of a tile at a time through the layers, 121
+// VGPRs) take the same time.
 // One kernel for inference (MODE_C2P), plain forward (MODE_FWD, outputs y)
 // and the training forward (MODE_TRAIN: y, network inputs h0, pre-activations
 // z1..z3 and rounded activations h1..h3, all [feature][state]).
@@ -255,6 +284,7 @@ __global__ __launch_bounds__(BLOCK, 3) void k_mlp(NetArgs net, C2pArgs ca, const
   __shared__ float sBias[BS_N];
   __shared__ h16x8 sX[4][64];
   __shared__ float2 sY[4][64];
+  __shared__ double sU[MODE == MODE_C2P ? 4 : 1][8][64];   // this tile's states during the layers
 
   if (MODE == MODE_C2P && ca.in_step && (ca.S->run_crashed || ca.S->temp_check)) return;   // block-uniform
   {  // weights to LDS
@@ -274,30 +304,51 @@ __global__ __launch_bounds__(BLOCK, 3) void k_mlp(NetArgs net, C2pArgs ca, const
   }
   __syncthreads();
 
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
   const long long ntiles = (n + 63) / 64;
-  double g33 = 1.0, gm = 1.0;
+  double g33 = 1.0, ig33 = 1.0, gm = 1.0;
   if (MODE == MODE_C2P) {
     const Metric M = make_metric(ca.coordinates, ca.S->t);
     g33 = M.g3;
+    ig33 = M.ig3;
     gm = M.gm;
   }
 
-  for (long long t0 = (long long)blockIdx.x * 4; t0 < ntiles; t0 += (long long)gridDim.x * 4) {
+  // The next tile's states are loaded while this one is in the layers and the
+  // refinement; the registers for them are the ones of this tile's states,
+  // which wait in LDS (sU) from the features to the refinement.  A lane past
+  // the last state loads that state again and stores nothing.
+  const long long t00 = (long long)blockIdx.x * 4;
+  double nu[8];
+  auto fetch = [&](long long tile) {
+    const long long s0 = 64 * (tile < ntiles ? tile : ntiles - 1);
+    const double* p = Ub + off + s0;
+    const unsigned l = s0 + lane < n ? lane : (unsigned)(n - 1 - s0);
+#pragma unroll
+    for (int k = 0; k < 8; k++) nu[k] = __builtin_nontemporal_load(p + k * stride + l);
+  };
+  auto park = [&] {
+#pragma unroll
+    for (int k = 0; k < 8; k++) sU[w][k][lane] = gm * nu[k];
+  };
+  if (MODE == MODE_C2P && t00 < ntiles) {
+    fetch(t00 + w);
+    park();
+  }
+
+  for (long long t0 = t00; t0 < ntiles; t0 += (long long)gridDim.x * 4) {
     const long long tile = t0 + w;
     const long long s = tile * 64 + lane;
-    const bool valid = (tile < ntiles) && (s < n);
-    double u[8];
-    if (valid) {
-#pragma unroll
-      for (int k = 0; k < 8; k++) u[k] = gm * Ub[k * stride + off + s];
-    } else {
-      u[0] = 1.0; u[1] = 0.0; u[2] = 0.0; u[3] = 0.0; u[4] = 1.0; u[5] = 0.0; u[6] = 0.0; u[7] = 0.0;
-    }
+    const bool valid = s < n;
     {
+      if (MODE != MODE_C2P) fetch(tile);
+      double u[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) u[k] = MODE == MODE_C2P ? sU[w][k][lane] : nu[k];
+      if (MODE == MODE_C2P) fetch(tile + (long long)gridDim.x * 4);
       float x[8];
-      features(u, g33, x);
+      features(u, g33, ig33, x);
       h16x8 xb;
 #pragma unroll
       for (int k = 0; k < 8; k++) xb[k] = (_Float16)x[k];
@@ -415,13 +466,16 @@ __global__ __launch_bounds__(BLOCK, 3) void k_mlp(NetArgs net, C2pArgs ca, const
       if (g == 0) sY[w][16 * q + c] = make_float2(y4[q][0], y4[q][1]);
     wave_sync();
     const float y1 = sY[w][lane].y;
-    double v[8];
-    const bool ok = valid && refine(u, y1, g33, ca.iters, ca.tol, v);
+    double u[8], v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) u[k] = sU[w][k][lane];
+    const bool ok = refine(u, y1, g33, ig33, ca.iters, ca.tol, v) && valid;
+    park();
     if (ok) {
 #pragma unroll
-      for (int k = 0; k < 8; k++) Vb[k * stride + off + s] = v[k];
+      for (int k = 0; k < 8; k++) __builtin_nontemporal_store(v[k], Vb + (k * stride + off + 64 * tile) + (unsigned)lane);
       if (NVU == 9) Vb[8 * stride + off + s] = Ub[8 * stride + off + s];
-      if (status) status[off + s] = 0;
+      if (status) (status + (off + 64 * tile))[(unsigned)lane] = 0;
     }
     const bool bad = valid && !ok;
     const unsigned long long mask = __ballot(bad);
