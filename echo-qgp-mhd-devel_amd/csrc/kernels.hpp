@@ -291,11 +291,13 @@ constexpr int flux_group() {
 }
 
 // Launch bounds: three waves per SIMD (at most 168 VGPRs), which the viscous
-// resistive system (NV = 19, 160 VGPRs, 51 KB of LDS per block) takes; the
-// smaller systems run four (114 VGPRs, 37 KB for NV = 12), hydro six.
+// resistive system (NV = 19, 152 VGPRs, 51 KB of LDS per block) takes; the
+// smaller systems run four (102 to 116 VGPRs, 37 KB for NV = 12), hydro six.
+// A sweep of 192 x 192 x 128 cells takes 0.50 to 0.55 ms for NV = 19 and 0.32
+// to 0.36 for NV = 12 (0.88 and 0.52 by interface, without the staging).
 // With a second staging buffer (one barrier per group instead of two) the
-// LDS allowed two and three: 0.62 instead of 0.54 ms a sweep for NV = 19,
-// 0.40 instead of 0.36 for NV = 12, on 192 x 192 x 128 cells.
+// LDS allowed two and three waves: 0.62 instead of 0.54 ms and 0.40 instead
+// of 0.36, measured before the carried components' HLL weights.
 template <int SYS>
 constexpr int flux_waves() { return SysT<SYS>::NV > 5 ? 3 : 6; }
 
@@ -801,13 +803,15 @@ struct StageArgs {
 };
 static_assert(UPDATE_BLOCK / 64 == 4, "the update's block maximum");
 
-// Waves per SIMD that the update's registers allow for (192 x 192 x 128
-// cells).  Three (168 VGPRs) for viscous hydro and ideal MHD, without
-// spills: ideal MHD 0.195 ms instead of 0.208 at two on 160 x 150 x 70 cells,
-// viscous hydro the same at both; at four both spill (viscous hydro 1.29
-// instead of 0.93 ms).  The viscous resistive RK update spills 164 bytes at
-// three (0.524 instead of 0.483 ms on 131 x 117 x 75 cells); its IMEX stages
-// 2 and 3 only 60, which pays (1.48 instead of 1.52 ms a launch).
+// Waves per SIMD that the update's registers allow for, each choice timed
+// against its neighbours when it was made.  At least three (168 VGPRs) for
+// viscous hydro and ideal MHD: ideal MHD 0.195 ms instead of 0.208 at two on
+// 160 x 150 x 70 cells (with algorithm 5 alone its 120 VGPRs run four, 0.166
+// now), viscous hydro the same at both (0.83 now on 192 x 192 x 128: 4.35 GB,
+// 5.2 TB/s); bounded for four, viscous hydro spills (1.29 instead of 0.93 ms).
+// The viscous resistive RK update spills 164 bytes at three (0.524 instead of
+// 0.483 ms on 131 x 117 x 75 cells; 0.39 now at two); its IMEX stages 2 and 3
+// only 20, which pays (1.48 instead of 1.52 ms a launch; 1.24 and 1.40 now).
 template <int SYS>
 constexpr int update_waves() { return SYS == SYS_VRMHD ? 2 : SysT<SYS>::NV > 5 ? 3 : 4; }
 template <int SYS, int STAGE>
@@ -826,9 +830,9 @@ constexpr int imex_update_waves() { return SYS == SYS_VRMHD ? (STAGE == 4 ? 2 : 
 //
 // ALGO: the ideal-MHD inversion algorithm when the launch knows it (5), else 0
 // (read from the arguments).  With all algorithms in one kernel the ideal-MHD
-// update needs 178 VGPRs, two waves per SIMD; with algorithm 5 alone it runs
-// three (0.195 instead of 0.288 ms a launch on 160 x 150 x 70
-// cells, with the divisions taken out of algorithm 5).
+// update needed 178 VGPRs, two waves per SIMD; with algorithm 5 alone it takes
+// 120 and runs four (0.166 ms a launch on 160 x 150 x 70 cells, 0.288 before,
+// with the divisions taken out of algorithm 5 and the tiles of update_cell).
 //
 // CFL: the update of a first stage on a small grid also forms dt from the
 // sweeps' block maxima (at most CFL_IN_UPDATE of them, up to four loads a

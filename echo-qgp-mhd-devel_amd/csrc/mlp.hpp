@@ -258,7 +258,7 @@ struct C2pArgs {
 // What bounds it: the SIMDs' issue.  Counted over 2^24 states, vector
 // instructions hold a SIMD for 68 % of the cycles and MFMA for another 32 %, and
 // the kernel takes what instructions are taken out of it: .67 ms with two
-// reciprocals an iterate, divisions and addresses per lane; .60 ms (2.2 GB, 3.6
+// reciprocals an iterate, divisions and addresses per lane; .58 ms (2.2 GB, 3.8
 // TB/s; a streaming copy's time would be .35) with the one-reciprocal residual
 // (e3p_w) and a wave's tile at a scalar base.  States are read and written
 // once, past the caches (nontemporal, .02 ms).
