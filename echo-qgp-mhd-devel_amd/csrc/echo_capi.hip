@@ -422,6 +422,9 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
   g->nf[1] = (long long)c.nx * (c.ny + 1) * c.nz;
   g->nf[2] = (long long)c.nx * c.ny * (c.nz + 1);
   g->active[0] = c.nx > 1; g->active[1] = c.ny > 1; g->active[2] = c.nz > 1;
+  // a grid without a sweep has no kernel that would hold its stages back after
+  // a failed one (echo_steps), so its steps hold the repairs from the start
+  g->repairs = !g->active[0] && !g->active[1] && !g->active[2];
   long long nb_cap = 1 + (long long)nblocks(g->N, CHECK_BLOCK);
   // what echo_get_tile reports until a shape is set or tuned; the sweeps take
   // the shape of flux_tx until then
