@@ -86,6 +86,19 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
+// 1/x and x / d for every operand, as the division gives them: the step makes a
+// NaN of inf * 0 where the hardware reciprocal is infinite (0, denormals) or
+// zero (infinities), and there the division itself is taken (a branch that no
+// wave of regular states enters)
+__device__ __forceinline__ double rcp_any(double x) {
+  const double r = rcp_nr(x);
+  return r == r ? r : 1. / x;
+}
+__device__ __forceinline__ double quot_any(double x, double d) {
+  const double r = rcp_nr(d);
+  return r == r ? x * r : x / d;
+}
+
 // 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
 // hardware reciprocal square root and one cubic step r (1 + e/2 + 3 e^2/8),
 // e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
@@ -1139,17 +1152,23 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
   // and the Newton step still uses them (system.f90:534-538, 627-631);
   // before the first successful call the reference reads uninitialised
   // locals there.  They start at 0 here.
-  double pr, w = 0., iw = 0., v2 = 0., glf, rh = 0., en, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
+  // The quotients by w hold for every w (rcp_any): a state without a finite
+  // energy ends with the error of its lookups, as with divisions, and not as a
+  // NaN that counts as inverted.
+  double pr, w = 0., v2 = 0., glf, rh = 0., en, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
   EosBracket br;
+  // drho/dp, which only the ideal gas's pressure needs; for the others (dp/drho
+  // = 0) it is 0, or NaN for a density that is not finite, which then ends as
+  // such in every primitive
+  const double drh0 = 0. * d;
   if constexpr (!VISC) {
     pr = v[KPR];
     for (int iter = 1; iter <= 100; iter++) {
       w = et + pr;
-      iw = rcp_nr(w);
-      v2 = s2 * (iw * iw);
-      if (v2 >= 1. || (w == 0. && s2 > 0.)) return 777;
+      v2 = quot_any(s2, w * w);
+      if (v2 >= 1.) return 777;
       en = w * (1. - v2) - pr;
-      double drh = 0.;   // dp/drho drho/dp: the ideal gas only
+      double drh = drh0;
       if (E.eqstate == 2) {
         glf = 1. / sqrt(1. - v2);
         rh = d / glf;
@@ -1163,6 +1182,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
       pr = pr + dpr;
     }
     if (E.eqstate != 2) rh = d * sqrt(1. - v2);
+    const double iw = rcp_any(w);
     v[KRH] = rh;
     v[KVX] = sx * iw;
     v[KVY] = sy * iw;
@@ -1175,9 +1195,8 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
 #pragma unroll
     for (int k = 0; k < NV; k++) uin[k] = gm * u[k];
     d = uin[KRH];
-    const double id = 1. / d;
 #pragma unroll
-    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = uin[k] * id;
+    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = quot_any(uin[k], d);
     double vx = v[KVX], vy = v[KVY], vz = v[KVZ];
 #pragma unroll
     for (int k = 0; k < NV; k++) vprim[k] = v[k];
@@ -1195,11 +1214,10 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
       pr = v[KPR];
       for (int ip = 1; ip <= 100; ip++) {
         w = en1 + pr;
-        iw = rcp_nr(w);
-        v2 = s2 * (iw * iw);
-        if (v2 >= 1. || (w == 0. && s2 > 0.)) return 107;
+        v2 = quot_any(s2, w * w);
+        if (v2 >= 1.) return 107;
         en = w * (1. - v2) - pr - vprim[KPIBU];
-        double drh = 0.;   // dp/drho drho/dp: the ideal gas only
+        double drh = drh0;
         if (E.eqstate == 2) {
           glf = 1. / sqrt(1. - v2);
           rh = d / glf;
@@ -1212,7 +1230,7 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
         if (fabs(dpr) < tol * pr) break;
         pr = pr + dpr;
       }
-      iw = rcp_nr(en1 + pr);
+      const double iw = rcp_any(en1 + pr);
       vx = sx * iw; if (fabs(vx) < eps) vx = 0.;
       vy = sy * iw; if (fabs(vy) < eps) vy = 0.;
       vz = sz * iw; if (fabs(vz) < eps) vz = 0.;
