@@ -40,11 +40,12 @@ static int flux_tx(const echo_config& c, int d, int ty);
 static unsigned sweep_blocks(const echo_grid* g, int d) { return g->active[d] ? (unsigned)g->nb[d] : 0u; }
 
 // flux launch of the sweeps in `dirs` (bit d for direction d) with the grid's
-// tile shapes
+// tile shapes; their speeds go to row `speeds` of aflux
 template <int SYS, bool ZZ>
-static void launch_flux(echo_grid* g, unsigned dirs, int irk) {
+static void launch_flux(echo_grid* g, unsigned dirs, int irk, int speeds) {
   FluxBufs b;
   b.irk = irk;
+  b.speeds = speeds;
   unsigned n = 0, off = 0;
   for (int d = 0; d < 3; d++) {
     b.partial[d] = g->partial + off;
@@ -71,10 +72,10 @@ static void launch_flux(echo_grid* g, unsigned dirs, int irk) {
 // the events ev[0..3].
 template <int SYS, bool ZZ>
 static void launch_sweeps(echo_grid* g, int irk) {
-  if (!g->timing) return launch_flux<SYS, ZZ>(g, 7u, irk);
+  if (!g->timing) return launch_flux<SYS, ZZ>(g, 7u, irk, irk - 1);
   for (int d = 0; d < 3; d++) {
     hipEventRecord(g->ev[d], g->stream);
-    launch_flux<SYS, ZZ>(g, 1u << d, irk);
+    launch_flux<SYS, ZZ>(g, 1u << d, irk, irk - 1);
   }
   hipEventRecord(g->ev[3], g->stream);
 }
@@ -238,9 +239,11 @@ static void enqueue_stage(echo_grid* g, int irk, bool fixup = true) {
   });
 }
 
-// one flux sweep (direction d = 0, 1, 2) with the current tile shape
+// one flux sweep (direction d = 0, 1, 2) of the tuner with the current tile shape
 static void enqueue_flux(echo_grid* g, int d) {
-  dispatch_sys(g->cfg, [&](auto sys, auto zz) { launch_flux<decltype(sys)::value, decltype(zz)::value>(g, 1u << d, 1); });
+  dispatch_sys(g->cfg, [&](auto sys, auto zz) {
+    launch_flux<decltype(sys)::value, decltype(zz)::value>(g, 1u << d, 1, AFLUX_TUNER);
+  });
 }
 
 static int set_tile(echo_grid* g, int d, int ty) {

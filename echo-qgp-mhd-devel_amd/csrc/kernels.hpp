@@ -23,7 +23,7 @@ struct DevScalars {
   double g3, gp, gm, ig3;  // the metric at t (set_metric)
   double smooth_pressure, dtout, tmax;
   double temp_end;         // check_temp threshold (<= 0: no check)
-  double aflux[4][3];      // per stage: max(ap, am) at the last interface of each sweep
+  double aflux[5][3];      // per stage: max(ap, am) at the last interface of each sweep (AFLUX_TUNER: no stage's)
   double check_max;        // max temperature (or energy density) of the last check
   long long nrepair;       // cells repaired by k_fixup since set-up
   long long nfallback;     // states the learned inversion in the step left to the plain solver
@@ -50,6 +50,8 @@ __device__ __forceinline__ Metric cur_metric(const DevScalars* S) {
   m.t = S->t; m.g3 = S->g3; m.gp = S->gp; m.gm = S->gm; m.ig3 = S->ig3;
   return m;
 }
+
+constexpr int AFLUX_TUNER = 4;   // the tuner's sweeps, which may run between an event's stages
 
 enum { CRASH_NONE = 0, CRASH_REPAIR = 1, CRASH_FLUX = 2, CRASH_SOURCE = 3 };
 
@@ -317,7 +319,8 @@ struct FluxBufs {
   double* partial[3];
   unsigned nb[3];
   int tx[3];
-  int irk;   // stage
+  int irk;     // stage
+  int speeds;  // row of aflux
 };
 
 template <int SYS>
@@ -332,7 +335,7 @@ struct FluxLds {
 template <int DIR, int REC, int SYS, bool ZZ>
 __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __restrict__ V, double* __restrict__ F,
                                            double* __restrict__ L, double* __restrict__ partial, unsigned block,
-                                           unsigned nblocks, int tx, int irk, FluxLds<SYS>& lds) {
+                                           unsigned nblocks, int tx, int irk, int speeds, FluxLds<SYS>& lds) {
   constexpr bool VISC = SysT<SYS>::VISC;
   constexpr int NV = SysT<SYS>::NV;
   const int nx = a.nx, ny = a.ny, nz = a.nz;
@@ -612,7 +615,7 @@ __device__ __forceinline__ void flux_block(const GridArgs& a, const double* __re
       double am = dmax(dmax(0., -vfl1), -vfr1);
       amax = dmax(ap, am);
       // aflux(dir) keeps the last interface of the sweep (work.f90:217,310,401)
-      if (f == nf - 1) a.S->aflux[irk - 1][DIR - 1] = amax;
+      if (f == nf - 1) a.S->aflux[speeds][DIR - 1] = amax;
       double a1 = (ap == 0.0 && am == 0.0) ? 1. : rcp_nr(ap + am);
       // resistive: B, E and psi with the speed of light (coordinate speed
       // 1 / sqrt(g_dir))
@@ -670,12 +673,13 @@ __global__ __launch_bounds__(FLUX_BLOCK, flux_waves<SYS>()) void k_flux(GridArgs
     return;
   }
   unsigned i = blockIdx.x;
-  if (i < b.nb[0]) return flux_block<1, REC, SYS, ZZ>(a, V, b.F[0], b.L[0], b.partial[0], i, b.nb[0], b.tx[0], b.irk, lds);
+  if (i < b.nb[0])
+    return flux_block<1, REC, SYS, ZZ>(a, V, b.F[0], b.L[0], b.partial[0], i, b.nb[0], b.tx[0], b.irk, b.speeds, lds);
   i -= b.nb[0];
   if (i < b.nb[1])
-    return flux_block<2, REC, SYS, ZZ>(a, V, b.F[1], b.L[1], b.partial[1], i, b.nb[1], b.tx[1], b.irk, lds);
+    return flux_block<2, REC, SYS, ZZ>(a, V, b.F[1], b.L[1], b.partial[1], i, b.nb[1], b.tx[1], b.irk, b.speeds, lds);
   i -= b.nb[1];
-  flux_block<3, REC, SYS, ZZ>(a, V, b.F[2], b.L[2], b.partial[2], i, b.nb[2], b.tx[2], b.irk, lds);
+  flux_block<3, REC, SYS, ZZ>(a, V, b.F[2], b.L[2], b.partial[2], i, b.nb[2], b.tx[2], b.irk, b.speeds, lds);
 }
 
 // ---------------------------------------------------------------------------

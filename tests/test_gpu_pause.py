@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from echoamd.initial import make_config
-from scenarios import force_superluminal
+from scenarios import force_superluminal, mhd_fireball3d
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +56,28 @@ def test_single_cell(coordinates, viscosity, nrk):
     ref = run("stages")
     assert ref[2] == nrk and ref[3]["iter"] == 5
     _same(run("call"), ref)
+
+
+def test_ensemble_tune_between_stages():
+    """The ensemble's tuner may run while an event is inside a step; its sweeps
+    change nothing of that step, the cleaning speed of the next stage (the
+    speeds of this one's sweeps) included."""
+    from echoamd import Ensemble
+    ic, rc, v0 = mhd_fireball3d(20, 18, 12)
+    v0[1] *= 0.1      # the y sweep, which the tuner runs, has the largest speed
+
+    def run(tune):
+        ens = Ensemble([(ic, rc)])
+        g = ens.grids[0]
+        assert g.init_from_prim(v0) == 0
+        ens.steps(2)
+        for irk in (1, 2, 3):
+            g.rk_stage(irk)
+            if tune and irk < 3:
+                ens.tune(reps=1)
+        g.end_step()
+        out = g.state() + (g.repairs(), g.scalars())
+        ens.close()
+        return out
+
+    _same(run(True), run(False))
