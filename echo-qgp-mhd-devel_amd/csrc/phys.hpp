@@ -86,17 +86,13 @@ __device__ __forceinline__ double rcp_nr(double x) {
   return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// 1/x and x / d for every operand, as the division gives them: the step makes a
-// NaN of inf * 0 where the hardware reciprocal is infinite (0, denormals) or
-// zero (infinities), and there the division itself is taken (a branch that no
-// wave of regular states enters)
+// 1/x for every operand, as the division gives it: the step makes a NaN of
+// inf * 0 where the hardware reciprocal is infinite (0, denormals) or zero
+// (infinities), and there the division itself is taken (a branch that no wave of
+// regular states enters)
 __device__ __forceinline__ double rcp_any(double x) {
   const double r = rcp_nr(x);
   return r == r ? r : 1. / x;
-}
-__device__ __forceinline__ double quot_any(double x, double d) {
-  const double r = rcp_nr(d);
-  return r == r ? x * r : x / d;
 }
 
 // 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
@@ -1156,9 +1152,10 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
   // and the Newton step still uses them (system.f90:534-538, 627-631);
   // before the first successful call the reference reads uninitialised
   // locals there.  They start at 0 here.
-  // The quotients by w hold for every w (rcp_any): a state without a finite
-  // energy ends with the error of its lookups, as with divisions, and not as a
-  // NaN that counts as inverted.
+  // The quotients by w hold for every w: a state without a finite energy ends
+  // with the error of its lookups, as with divisions, and not as a NaN that
+  // counts as inverted.  Where s2 (1/w)^2 is no number below 1 (a superluminal
+  // state, or a reciprocal out of range) the division s2 / w^2 decides.
   double pr, w = 0., v2 = 0., glf, rh = 0., en, dprdrh = 0., dprden = 0., f, df, dpr, pr_eos = 0.;
   EosBracket br;
   // drho/dp, which only the ideal gas's pressure needs; for the others (dp/drho
@@ -1169,8 +1166,12 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
     pr = v[KPR];
     for (int iter = 1; iter <= 100; iter++) {
       w = et + pr;
-      v2 = quot_any(s2, w * w);
-      if (v2 >= 1.) return 777;
+      const double ir = rcp_nr(w);
+      v2 = s2 * (ir * ir);
+      if (!(v2 < 1.)) {
+        v2 = s2 / (w * w);
+        if (v2 >= 1.) return 777;
+      }
       en = w * (1. - v2) - pr;
       double drh = drh0;
       if (E.eqstate == 2) {
@@ -1199,8 +1200,13 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
 #pragma unroll
     for (int k = 0; k < NV; k++) uin[k] = gm * u[k];
     d = uin[KRH];
+    const double id = 1. / d;
 #pragma unroll
-    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = quot_any(uin[k], d);
+    for (int k = KPIBU; k <= KPIZZ; k++) v[k] = uin[k] * id;
+    if (__builtin_isinf(id)) {   // a density of 0 or a denormal one
+#pragma unroll
+      for (int k = KPIBU; k <= KPIZZ; k++) v[k] = uin[k] / d;
+    }
     double vx = v[KVX], vy = v[KVY], vz = v[KVZ];
 #pragma unroll
     for (int k = 0; k < NV; k++) vprim[k] = v[k];
@@ -1218,8 +1224,12 @@ __device__ __forceinline__ int cons2prim(const Eos& E, const Metric& M, const do
       pr = v[KPR];
       for (int ip = 1; ip <= 100; ip++) {
         w = en1 + pr;
-        v2 = quot_any(s2, w * w);
-        if (v2 >= 1.) return 107;
+        const double ir = rcp_nr(w);
+        v2 = s2 * (ir * ir);
+        if (!(v2 < 1.)) {
+          v2 = s2 / (w * w);
+          if (v2 >= 1.) return 107;
+        }
         en = w * (1. - v2) - pr - vprim[KPIBU];
         double drh = drh0;
         if (E.eqstate == 2) {
