@@ -885,8 +885,14 @@ int echo_end_step(echo_grid* g) {
   return read_crash(g);
 }
 
-// n replays of the captured step, with or without the repairs
+// n steps, with or without the repairs: replays of the captured step, after
+// PLAIN_STEPS plain launches behind which its capture and instantiation (50 us,
+// 0.4 ms for a size the runtime holds no memory for) pass unnoticed
+constexpr int PLAIN_STEPS = 3;
+
 static int launch_steps(echo_grid* g, int n, bool fixup) {
+  for (; n > 0 && !g->gexec && g->plain_steps < PLAIN_STEPS; n--, g->plain_steps++) enqueue_step(g, fixup);
+  HIPCHECK(hipGetLastError());
   if (n <= 0) return 0;
   if (!g->gexec) {
     HIPCHECK(hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal));
@@ -900,6 +906,9 @@ static int launch_steps(echo_grid* g, int n, bool fixup) {
   HIPCHECK(hipGetLastError());
   return 0;
 }
+
+// steps without repairs between two looks for one that needs them, at first
+constexpr int STEPS_UNSEEN = 32;
 
 int echo_steps(echo_grid* g, int32_t nsteps) {
   if (!g) return fail(ECHO_E_ARG, "null argument");
@@ -939,13 +948,30 @@ int echo_steps(echo_grid* g, int32_t nsteps) {
   // failed cells return at once (paused), the step is finished here with the
   // repair, and from then on the grid's steps hold the repairs.  IMEX steps
   // and the learned inversion always do.
+  //
+  // What was queued behind a step that paused is queued again, and an empty
+  // replay costs 25 us where a step of a small grid takes 42, so the call looks
+  // for it on the way: after the grid's first step (before a graph without
+  // repairs is captured for nothing), then after 32 steps, 64, 128, ...; a look
+  // idles the GPU for some 25 us, and fewer than twice a chunk's steps go without
+  // one.  400 steps of 10 x 10 x 8 cells that need repairs from their first take
+  // 18.9 ms, 18.5 with the repairs in place before (28.2 when all 400 were queued
+  // without them first); 20 steps 1.16 and 0.97 ms (2.16).
   int left = nsteps;
-  if (!g->repairs && g->cfg.nrk != 4 && !g->net) {
+  int chunk = g->clean_step ? STEPS_UNSEEN : 1;
+  while (left > 0 && !g->repairs && g->cfg.nrk != 4 && !g->net) {
+    const int n = left < 2 * chunk ? left : chunk;
     const int first = g->iter;
-    if (int e = launch_steps(g, left, false)) return e;
+    if (int e = launch_steps(g, n, false)) return e;
     DevScalars S;
     if (int e = read_scalars(g, S)) return e;
-    if (S.nfail == 0) return crash_of(g, S);
+    if (S.nfail == 0) {
+      g->clean_step = true;
+      left -= n;
+      if (left <= 0 || S.run_crashed || S.temp_check) return crash_of(g, S);
+      chunk = chunk == 1 ? STEPS_UNSEEN : 2 * chunk;
+      continue;
+    }
     g->repairs = true;
     drop_graph(g);
     enqueue_fixup(g, S.fail_stage);

@@ -69,6 +69,8 @@ struct echo_grid {
   int next_stage = 1;
   int iter = 0;               // steps taken, as of the last read of the scalars
   bool repairs = false;       // the captured step holds the con2prim repairs (echo_steps)
+  bool clean_step = false;    // a step has gone without needing them
+  int plain_steps = 0;        // steps launched since the graph was dropped (launch_steps)
   int tile[3] = {1, 1, 1};    // flux tile shape per sweep (echo_set_tile)
   bool tile_set = false;      // set or tuned; until then flux_tx chooses
   bool owns_scratch = true;   // F, L, partial (shared inside an ensemble)
@@ -121,6 +123,7 @@ void enqueue_net_c2p(echo_grid* g, const double* U);
 
 // forget the grid's captured step (rebuilt at the next echo_steps)
 inline void drop_graph(echo_grid* g) {
+  g->plain_steps = 0;
   if (g->gexec) hipGraphExecDestroy(g->gexec);
   if (g->graph) hipGraphDestroy(g->graph);
   g->gexec = nullptr;

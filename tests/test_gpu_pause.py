@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from echoamd.initial import make_config
-from scenarios import force_superluminal, mhd_fireball3d
+from scenarios import force_superluminal, forced_background, mhd_fireball3d
 
 pytestmark = pytest.mark.gpu
 
@@ -81,3 +81,109 @@ def test_ensemble_tune_between_stages():
         return out
 
     _same(run(True), run(False))
+
+
+def _fast_cells(v_eta, maxdt, nrk, mhd=0, viscosity=0, smooth_temp=0.0, pbg=0.05):
+    """A Bjorken grid with two cells at v^eta = v_eta, whose own v^2 passes 1 as
+    tau grows: the first inversions fail some steps after the start."""
+    ic, rc, v = forced_background(eqstate=1, rec="TVD2", pbg=pbg, coordinates=2, viscosity=viscosity,
+                                  smooth_temp=smooth_temp)
+    for (z, y, x) in ((4, 5, 5), (3, 4, 6)):
+        v[1, z, y, x], v[2, z, y, x], v[3, z, y, x] = 0.05, 0.0, v_eta
+        v[5:, z, y, x] = 0.0
+    # a hot corner, whose cooling the stop check follows
+    v[4, :2, :3, :3] *= 20.0
+    ic, rc = ic.copy(), rc.copy()
+    rc[8], ic[10] = maxdt, nrk
+    if mhd:
+        ic[6], ic[7], ic[12] = 1, 1, 5
+        v = np.concatenate([v, np.zeros((4,) + v.shape[1:])])
+        v[5], v[6], v[7] = 0.02, 0.03, 0.01
+    return ic, rc, v
+
+
+# arguments, steps, the first step that fails and its stage (both from 1)
+LATE = {
+    "hydro-rk2": (dict(v_eta=0.992, maxdt=0.0009, nrk=2), 40, 23, 1),
+    "hydro-rk3": (dict(v_eta=0.993, maxdt=0.001, nrk=3), 75, 48, 1),
+    "mhd-rk2-last-stage": (dict(v_eta=0.991, maxdt=0.0009, nrk=2, mhd=1), 80, 59, 2),
+    "mhd-rk3-middle-stage": (dict(v_eta=0.994, maxdt=0.0012, nrk=3, mhd=1), 12, 3, 2),
+    "viscous-rk2": (dict(v_eta=0.95, maxdt=0.02, nrk=2, viscosity=1, pbg=0.3), 12, 2, 1),
+    "viscous-smooth-rk3": (dict(v_eta=0.95, maxdt=0.02, nrk=3, viscosity=1, pbg=0.3, smooth_temp=0.15), 12, 2, 1),
+}
+
+
+@pytest.mark.parametrize("hooks", ["plain", "dump and stop"])
+@pytest.mark.parametrize("name", list(LATE))
+def test_first_failure_inside_a_call(name, hooks, tmp_path):
+    """One call whose first failed inversion comes after clean steps of the same
+    call, in each stage, with the dump's copies and a stop check that ends the
+    run after the repair in between."""
+    from echoamd import EchoGrid
+    kw, n, step, stage = LATE[name]
+    ic, rc, v0 = _fast_cells(**kw)
+
+    def grid(e_end):
+        g = EchoGrid(ic, rc)
+        assert g.init_from_prim(v0) == 0
+        if hooks != "plain":
+            g.set_dump(True)
+            g.set_stop(e_end, freeze_type=1)
+        return g
+
+    # where the run fails first, and what the stop check sees at each step
+    g = grid(1e-30)
+    emax = []
+    for i in range(1, n + 1):
+        for irk in range(1, g.cfg.nrk + 1):
+            g.rk_stage(irk)
+            assert (g.repairs() > 0) == ((i, irk) >= (step, stage)), (i, irk)
+        g.end_step()
+        emax.append(g.stop_state()[1])
+    g.close()
+    # the check of step n - 2 is the first below this
+    e_end = 0.5 * (emax[n - 4] + emax[n - 3])
+    assert hooks == "plain" or (n - 3 > step and min(emax[:n - 3]) > e_end > emax[n - 3])
+
+    def run(how):
+        g = grid(e_end)
+        _advance(g, n, how)
+        out = g.state() + (g.repairs(), g.scalars())
+        if hooks != "plain":
+            f = tmp_path / how
+            g.dump(str(f), 1)
+            out += (f.read_bytes(), g.stop_state())
+        g.close()
+        return out
+
+    ref, call = run("stages"), run("call")
+    assert ref[3]["iter"] == (n if hooks == "plain" else n - 3)
+    _same(call, ref)
+    assert call[4:] == ref[4:]
+
+
+def test_failure_in_the_first_step_costs_no_second_run():
+    """A call of 400 steps that needs repairs from its first step takes about as
+    long as one on the same grid afterwards, whose steps hold the repairs from
+    their start (1.53 times as long when all 400 were queued without them
+    first)."""
+    import time
+    from echoamd import EchoGrid
+    ic, rc, v0 = forced_background()
+    rc = rc.copy()
+    rc[8] = 1e-3
+    ratio = []
+    for _ in range(7):
+        g = EchoGrid(ic, rc)
+        assert g.init_from_prim(v0) == 0
+        v, u = g.state()
+        g.upload(v, force_superluminal(u))
+        t = [time.perf_counter()]
+        for _ in range(2):
+            g.steps(400)
+            t.append(time.perf_counter())
+        assert g.repairs() > 0 and g.scalars()["iter"] == 800
+        g.close()
+        ratio.append((t[1] - t[0]) / (t[2] - t[1]))
+    print(f"\nfirst call over second: {np.round(sorted(ratio), 3)}", flush=True)
+    assert np.median(ratio) <= 1.25
