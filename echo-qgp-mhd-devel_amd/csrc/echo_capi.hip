@@ -28,13 +28,9 @@ static void rk_coeffs(int nrk, int irk, double& c1, double& c2) {
 // ---------------------------------------------------------------------------
 // kernel dispatch
 // ---------------------------------------------------------------------------
-// cells along x of a block of the y and z sweeps, for the tile rows 1, 2, 4
-// of echo_set_tile; 0: 16 or 32, by the number of blocks, where rows of 16
-// cells that do not start at a cache line (nx not a multiple of 16) count a
-// tenth more (192 x 192 x 128 cells: 0.36 at 16 against 0.38 ms at 32 a sweep;
-// 131 x 117 x 75: y, 72 against 85 blocks a plane, 0.168 against 0.180 ms; z,
-// 54 against 55, 0.186 against 0.168 ms)
-static int flux_tx(const echo_config& c, int d, int ty);
+// cells along x of a block of the y and z sweeps, for the tile rows 1, 2, 4 of
+// echo_set_tile
+static int flux_tx(int ty) { return ty == 1 ? 16 : ty == 2 ? 32 : 8; }
 
 // blocks of a sweep, 0 for a dimension with one cell
 static unsigned sweep_blocks(const echo_grid* g, int d) { return g->active[d] ? (unsigned)g->nb[d] : 0u; }
@@ -52,7 +48,7 @@ static void launch_flux(echo_grid* g, unsigned dirs, int irk, int speeds) {
     off += sweep_blocks(g, d);
     b.F[d] = g->F[d];
     b.L[d] = g->L[d];
-    b.tx[d] = flux_tx(g->cfg, d, g->tile_set ? g->tile[d] : 0);
+    b.tx[d] = flux_tx(g->tile[d]);
     b.nb[d] = dirs >> d & 1 ? sweep_blocks(g, d) : 0;
     n += b.nb[d];
   }
@@ -82,16 +78,20 @@ static void launch_sweeps(echo_grid* g, int irk) {
 
 // launch blocks of a sweep for tile shape ty (padded for xcd_block)
 static unsigned flux_blocks(const echo_config& c, int d, int ty) {
-  const int tx = flux_tx(c, d, ty);
+  const int tx = flux_tx(ty);
   long long t = d == 0 ? flux_tiles<1>(c.nx, c.ny, c.nz, tx, c.boundary_cond)
               : d == 1 ? flux_tiles<2>(c.nx, c.ny, c.nz, tx, c.boundary_cond)
                        : flux_tiles<3>(c.nx, c.ny, c.nz, tx, c.boundary_cond);
   return (unsigned)((t + NXCD - 1) / NXCD * NXCD);
 }
 
-static int flux_tx(const echo_config& c, int d, int ty) {
-  if (ty == 0) ty = d == 0 || flux_blocks(c, d, 1) * (c.nx % 16 ? 1.1 : 1.) <= flux_blocks(c, d, 2) ? 1 : 2;
-  return ty == 1 ? 16 : ty == 2 ? 32 : 8;
+// the shape a sweep takes until one is set or tuned: rows 1 or 2, by the number
+// of blocks, where rows of 16 cells that do not start at a cache line (nx not a
+// multiple of 16) count a tenth more (192 x 192 x 128 cells: 0.36 at 16 against
+// 0.38 ms at 32 a sweep; 131 x 117 x 75: y, 72 against 85 blocks a plane, 0.168
+// against 0.180 ms; z, 54 against 55, 0.186 against 0.168 ms)
+static int default_tile(const echo_config& c, int d) {
+  return d == 0 || flux_blocks(c, d, 1) * (c.nx % 16 ? 1.1 : 1.) <= flux_blocks(c, d, 2) ? 1 : 2;
 }
 
 static bool tiles_supported(const echo_config& c) { return c.recal == REC_WENO5 || c.recal == REC_PPM4; }
@@ -249,13 +249,9 @@ static void enqueue_flux(echo_grid* g, int d) {
 static int set_tile(echo_grid* g, int d, int ty) {
   if (d < 0 || d > 2) return fail(ECHO_E_ARG, "sweep index must be 0, 1 or 2");
   if (ty != 1 && ty != 2 && ty != 4) return fail(ECHO_E_ARG, "tile rows must be 1, 2 or 4");
-  if (ty != 1 && (d == 0 || !tiles_supported(g->cfg)))
-    return fail(ECHO_E_ARG, "tiled sweeps exist for y and z with WENO5 or PPM4");
-  if (!g->tile_set) {
-    // from here on every sweep takes the shape it reports
-    g->tile_set = true;
-    for (int k = 0; k < 3; k++) g->nb[k] = (int)flux_blocks(g->cfg, k, g->tile[k]);
-  }
+  // (the shape a grid starts with may always be set again)
+  if (ty != 1 && (d == 0 || !tiles_supported(g->cfg)) && ty != default_tile(g->cfg, d))
+    return fail(ECHO_E_ARG, "the tile shapes of the y and z sweeps are chosen with WENO5 or PPM4 only");
   g->tile[d] = ty;
   g->nb[d] = (int)flux_blocks(g->cfg, d, ty);
   drop_graph(g);
@@ -429,11 +425,9 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
   // a failed one (echo_steps), so its steps hold the repairs from the start
   g->repairs = !g->active[0] && !g->active[1] && !g->active[2];
   long long nb_cap = 1 + (long long)nblocks(g->N, CHECK_BLOCK);
-  // what echo_get_tile reports until a shape is set or tuned; the sweeps take
-  // the shape of flux_tx until then
-  if (tiles_supported(c) && c.nz > 1) g->tile[2] = 2;
   for (int d = 0; d < 3; d++) {
-    g->nb[d] = (int)flux_blocks(c, d, 0);
+    g->tile[d] = g->active[d] ? default_tile(c, d) : 1;
+    g->nb[d] = (int)flux_blocks(c, d, g->tile[d]);
     unsigned mx = 0;
     for (int ty : {1, 2, 4}) mx = std::max(mx, flux_blocks(c, d, ty));
     nb_cap += mx;

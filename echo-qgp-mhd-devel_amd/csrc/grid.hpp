@@ -71,8 +71,7 @@ struct echo_grid {
   bool repairs = false;       // the captured step holds the con2prim repairs (echo_steps)
   bool clean_step = false;    // a step has gone without needing them
   int plain_steps = 0;        // steps launched since the graph was dropped (launch_steps)
-  int tile[3] = {1, 1, 1};    // flux tile shape per sweep (echo_set_tile)
-  bool tile_set = false;      // set or tuned; until then flux_tx chooses
+  int tile[3] = {1, 1, 1};    // flux tile shape per sweep (default_tile, echo_set_tile)
   bool owns_scratch = true;   // F, L, partial (shared inside an ensemble)
   bool owns_stream = true;
   long long partial_cap = 0;  // doubles in partial

@@ -316,12 +316,13 @@ int echo_cons2prim_batch(echo_grid *g, const double *u, double *v, int32_t *stat
 /* Tile shape of the flux sweeps and its autotuner (no counterpart in the
  * reference, whose sweeps are pencil loops, evolve.f90:302-685).  The blocks
  * of a y or z sweep are 16 cells along x by 16 along the sweep with rows = 1,
- * 32 by 8 with rows = 2, 8 by 32 with rows = 4 (WENO5 and PPM4); results are
- * identical for every shape.  Until a shape is set or tuned the sweeps take
- * one of the first two by the grid's size.  echo_tune times each shape
- * on the current state (reps launches each) and keeps the fastest; ms
- * (optional, 9 doubles): per-launch times, [3*sweep + {0,1,2}] for rows
- * {1,2,4}. */
+ * 32 by 8 with rows = 2, 8 by 32 with rows = 4; results are identical for every
+ * shape.  A grid starts with one of the first two, by its size; echo_get_tile
+ * returns the shapes that the sweeps take.  With WENO5 and PPM4 any shape can be
+ * set; with the other reconstructions rows = 1 and the shape the grid started
+ * with.  echo_tune times each shape on the current state (reps launches each)
+ * and keeps the fastest; ms (optional, 9 doubles): per-launch times,
+ * [3*sweep + {0,1,2}] for rows {1,2,4}. */
 int echo_set_tile(echo_grid *g, int32_t sweep, int32_t rows);
 int echo_get_tile(const echo_grid *g, int32_t *rows);
 int echo_tune(echo_grid *g, int32_t reps, double *ms);
