@@ -85,13 +85,26 @@ static unsigned flux_blocks(const echo_config& c, int d, int ty) {
   return (unsigned)((t + NXCD - 1) / NXCD * NXCD);
 }
 
-// the shape a sweep takes until one is set or tuned: rows 1 or 2, by the number
-// of blocks, where rows of 16 cells that do not start at a cache line (nx not a
-// multiple of 16) count a tenth more (192 x 192 x 128 cells: 0.36 at 16 against
-// 0.38 ms at 32 a sweep; 131 x 117 x 75: y, 72 against 85 blocks a plane, 0.168
-// against 0.180 ms; z, 54 against 55, 0.186 against 0.168 ms)
+// variables of a grid
+static int num_vars(const echo_config& c) {
+  return c.mhd == 2 ? (c.viscosity ? 19 : 12) : c.mhd ? (c.divclean ? 9 : 8) : (c.viscosity ? 12 : 5);
+}
+
+// The shape a sweep takes until one is set or tuned: rows 1 (16 columns) or 2
+// (32), whichever has fewer blocks.  In the z sweeps of 12 variables a block of
+// 16 columns counts a twentieth more, of 19 a tenth, where rows of 16 cells do
+// not start at a cache line (nx not a multiple of 16).  Both shapes timed on 27
+// grids of 40 to 200 cells a side, nx % 16 from 2 to 14, block counts within
+// 30 % of each other, the choice costs on average over the better of the two
+//   y: 0.0, 0.0, 0.1, 0.0 and 1.4 % (hydro, ideal MHD, viscous hydro, resistive
+//      without and with viscosity);  z: 0.2, 0.5, 0.8, 0.9 and 1.4 %
+// With a tenth for every sweep it is 2 to 6 % for y and 7, 4, 1, 2 and 1 % for z;
+// without any, 13 % for the z sweeps of 19 variables.
 static int default_tile(const echo_config& c, int d) {
-  return d == 0 || flux_blocks(c, d, 1) * (c.nx % 16 ? 1.1 : 1.) <= flux_blocks(c, d, 2) ? 1 : 2;
+  if (d == 0) return 1;
+  const int nv = num_vars(c);
+  const double w = d == 2 && c.nx % 16 ? (nv > 12 ? 1.1 : nv > 9 ? 1.05 : 1.) : 1.;
+  return flux_blocks(c, d, 1) * w <= flux_blocks(c, d, 2) ? 1 : 2;
 }
 
 static bool tiles_supported(const echo_config& c) { return c.recal == REC_WENO5 || c.recal == REC_PPM4; }
@@ -415,7 +428,7 @@ static int grid_create(const echo_config* cfg, const double* eos_rows, int32_t n
   g->dev = device;
   hipError_t he = hipSetDevice(device);
   if (he != hipSuccess) { delete g; return fail(ECHO_E_HIP, "hipSetDevice: %s", hipGetErrorString(he)); }
-  g->nv = c.mhd == 2 ? (c.viscosity ? 19 : 12) : c.mhd ? (c.divclean ? 9 : 8) : (c.viscosity ? 12 : 5);
+  g->nv = num_vars(c);
   g->N = (long long)c.nx * c.ny * c.nz;
   g->nf[0] = (long long)(c.nx + 1) * c.ny * c.nz;
   g->nf[1] = (long long)c.nx * (c.ny + 1) * c.nz;

@@ -126,7 +126,10 @@ __device__ __forceinline__ double next_dt(const GridArgs& a, double amax) {
 
 // per-block speed maxima of a stage's sweeps (nb[d] of direction d, one after
 // the other), and how many of them a block of the first update reduces by
-// itself; grids with more leave it to k_cfl
+// itself; grids with more leave it to k_cfl.  Against k_cfl a step of 46 us
+// gains 1.4 us with 245 blocks (32 x 32 x 16 cells of hydro), one of 60 us 1.0
+// with 777; with 1100 to 2200 blocks the two are level, and with 5400, read by
+// every block of the update, it loses 7 us of 195.
 struct SpeedMax {
   const double* partial;
   unsigned nb[3];
