@@ -107,6 +107,9 @@ static int default_tile(const echo_config& c, int d) {
   return flux_blocks(c, d, 1) * w <= flux_blocks(c, d, 2) ? 1 : 2;
 }
 
+// whether echo_set_tile and the tuner offer a choice (k_flux takes any shape with
+// every reconstruction; the choice has always been these two's, and callers see
+// it refused for the others)
 static bool tiles_supported(const echo_config& c) { return c.recal == REC_WENO5 || c.recal == REC_PPM4; }
 
 // launch blocks of the cell updates (update_cell), padded for xcd_block

@@ -190,8 +190,8 @@ constexpr int NXCD = 8;   // MI355X: 8 XCDs, each with its own L2
 // space per XCD the hundred arrays of a cell update are read at eight distant
 // places each: viscous hydro update 0.889 instead of 0.833 ms, sweep x 0.337
 // instead of 0.322 ms, viscous resistive step 9.82 instead of 9.50 ms on
-// 192 x 192 x 128 cells; chunks of 1 to 64 lie within 1% of each other, 256
-// and more are slower again.)  A bijection on [0, nb); a last group that is
+// 192 x 192 x 128 cells; chunks of 1 to 128 lie within 1% of each other, 256
+// costs the sweeps and 512 the updates 2%.)  A bijection on [0, nb); a last group that is
 // not full stays in launch order.
 constexpr unsigned XCD_CHUNK = 16;
 __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
@@ -257,8 +257,10 @@ __device__ __forceinline__ int bc_map(int c0, int m, int bc) {
 // system.f90:1316-1583), and a per-block max of the fast speeds for the CFL
 // condition (evolve.f90:723-764).
 //
-// What bounds it: FP64 VALU issue (some 4 cycles per wave instruction, with
-// two or three waves per SIMD).  Reconstructing by cell instead of by
+// What bounds it: vector issue, three quarters of it FP64 (4 cycles a wave
+// instruction): it holds the SIMDs for 0.59 of the cycles at NV = 19 with three
+// waves each and 0.67 at NV = 12 with four, while half of the wave cycles wait;
+// the bytes go at 3.4 TB/s (192 x 192 x 128 cells, counted).  Reconstructing by cell instead of by
 // interface shares the smoothness indicators between a cell's two faces and
 // loads five cells per variable instead of six; the price is one row of
 // cells per tile whose upper face the next tile owns.

@@ -169,7 +169,7 @@ __device__ __forceinline__ void targets(const double* u, const double* v, double
 // alone (c3 = (3 + x)/4, c2 = B^2 (1 + x)/2 - U), from the network's W.  With
 // y = x W^2 = (S^2 W^2 + (2W + B^2)(S.B)^2) / (W + B^2)^2 it reads
 //   f = (3W/4 + B^2/2 - U) W^2 + (W/4 + B^2/2) y - (S.B)^2/2,
-// which takes one reciprocal an iterate.
+// which takes one reciprocal; the Newton step takes another.
 struct E3pInv {
   double S2, B2, SB, SB2;
   double h2;   // B^2 / 2
@@ -258,7 +258,7 @@ struct C2pArgs {
 // What bounds it: the SIMDs' issue.  Counted over 2^24 states, vector
 // instructions hold a SIMD for 68 % of the cycles and MFMA for another 32 %, and
 // the kernel takes what instructions are taken out of it: .67 ms with two
-// reciprocals an iterate, divisions and addresses per lane; .58 ms (2.2 GB, 3.8
+// reciprocals in the residual, divisions and addresses per lane; .58 ms (2.2 GB, 3.8
 // TB/s; a streaming copy's time would be .35) with the one-reciprocal residual
 // (e3p_w) and a wave's tile at a scalar base.  States are read and written
 // once, past the caches (nontemporal, .02 ms).

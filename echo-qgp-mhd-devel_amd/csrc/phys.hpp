@@ -95,9 +95,9 @@ __device__ __forceinline__ double rcp_any(double x) {
   return r == r ? r : 1. / x;
 }
 
-// 1/sqrt(x) for 0 < x <= 1 (Lorentz factors of subluminal states): the
-// hardware reciprocal square root and one cubic step r (1 + e/2 + 3 e^2/8),
-// e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
+// 1/sqrt(x) for 0 <= x in the normal range (Lorentz factors, squared distances,
+// sqrt_nr): the hardware reciprocal square root and one cubic step
+// r (1 + e/2 + 3 e^2/8), e = 1 - x r^2; x = 0 gives +inf as the IEEE form does.
 __device__ __forceinline__ double rsqrt_nr(double x) {
   const double r = __builtin_amdgcn_rsq(x);
   const double e = __builtin_fma(-(x * r), r, 1.0);
